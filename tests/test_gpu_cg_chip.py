@@ -1,0 +1,100 @@
+"""The plain CG solve as one launch (cg_chip.hip): boxes of every segment
+length, with remainders in each direction, at the smallest grids and on either
+side of the largest one that fits.  The bound is the solve's own stopping
+test, evaluated in numpy; FP64 rounding of the two residuals is far below it."""
+import numpy as np
+import pytest
+
+from tpls_amd import _lib
+from tpls_amd.case import Case, batch_step, set_batch_grouped
+from tpls_amd.config import CaseParams
+from tpls_amd.initial import make_initial
+
+pytestmark = pytest.mark.gpu
+
+
+def residual(x, b, h):
+    """b - mean(b) - A x on the interior cells (Neumann in x and z, periodic in y)."""
+    p = np.pad(x, ((1, 1), (0, 0), (1, 1)), mode="edge")
+    c = p[1:-1, :, 1:-1]
+    ax = (6 * c - p[:-2, :, 1:-1] - p[2:, :, 1:-1] - p[1:-1, :, :-2] - p[1:-1, :, 2:]
+          - np.roll(c, 1, 1) - np.roll(c, -1, 1)) / h ** 2
+    r = b - b.mean() - ax
+    return r - r.mean()
+
+
+@pytest.mark.parametrize("nx,ny,nz", [
+    (5, 4, 5), (7, 6, 9), (6, 4, 301), (303, 4, 7), (5, 130, 6), (33, 18, 29), (64, 16, 32), (96, 22, 41),
+    (128, 32, 64), (150, 46, 77), (129, 66, 65), (256, 64, 128), (211, 52, 190), (320, 96, 128)])
+def test_solution_meets_the_stopping_test(nx, ny, nz):
+    rng = np.random.default_rng(nx * 7 + ny * 3 + nz)
+    L, M, N, h = nx + 1, ny + 1, nz + 1, 1.0 / nz
+    rhs = np.asfortranarray(rng.standard_normal((L + 1, M + 1, N + 1)))
+    pres = np.asfortranarray(0.01 * rng.standard_normal((L + 1, M + 1, N + 1)))
+    u3 = np.zeros((L + 1, M + 1, N - 1), order="F")
+    b = -rhs[1:L, 1:M, 1:N]
+    mean0 = pres[1:L, 1:M, 1:N].mean()
+    rtol = 1e-8
+    its, rnorm, reason = _lib.pressure_solve(pres, rhs, u3, np.zeros(N - 1), L, M, N, h, h, h, 1e-4, rtol, 1e-50,
+                                             1e5, 10000)
+    assert reason == 2 and its > 0
+    x = pres[1:L, 1:M, 1:N]
+    rn, bn = np.linalg.norm(residual(x, b, h)), np.linalg.norm(b - b.mean())
+    # the recurrence's residual differs from the true one by rounding: about
+    # sqrt(iterations) eps |A| |x|
+    assert rn <= rtol * bn + 10 * np.sqrt(its) * 2.3e-16 * 12 / h ** 2 * np.linalg.norm(x)
+    # CG moves x by mean-free directions only
+    assert abs(x.mean() - mean0) <= 1e-10 * np.abs(x).max()
+    # the same call again gives the same bits
+    again = np.asfortranarray(0 * pres)
+    r1 = _lib.pressure_solve(again, rhs, u3, np.zeros(N - 1), L, M, N, h, h, h, 1e-4, rtol, 1e-50, 1e5, 10000)
+    twice = np.asfortranarray(0 * pres)
+    r2 = _lib.pressure_solve(twice, rhs, u3, np.zeros(N - 1), L, M, N, h, h, h, 1e-4, rtol, 1e-50, 1e5, 10000)
+    assert r1 == r2 and np.array_equal(again, twice)
+
+
+def test_iteration_limit_and_converged_guess():
+    """Stopping at maxits (KSP_DIVERGED_ITS), and no iteration at all from a converged guess."""
+    rng = np.random.default_rng(5)
+    nx, ny, nz = 40, 12, 26
+    L, M, N, h = nx + 1, ny + 1, nz + 1, 1.0 / nz
+    rhs = np.asfortranarray(rng.standard_normal((L + 1, M + 1, N + 1)))
+    pres = np.zeros((L + 1, M + 1, N + 1), order="F")
+    u3, inlet = np.zeros((L + 1, M + 1, N - 1), order="F"), np.zeros(N - 1)
+    a = (u3, inlet, L, M, N, h, h, h, 1e-4)
+    its, _, reason = _lib.pressure_solve(pres, rhs, *a, 1e-10, 1e-50, 1e5, 7)
+    assert (its, reason) == (7, -3)
+    its, _, reason = _lib.pressure_solve(pres, rhs, *a, 1e-10, 1e-50, 1e5, 10000)
+    assert reason == 2
+    before = pres.copy()
+    its, _, reason = _lib.pressure_solve(pres, rhs, *a, 1e-6, 1e-50, 1e5, 10000)
+    assert (its, reason) == (0, 2) and np.array_equal(pres, before)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2])
+def test_batch_equals_alone(mode):
+    """Plain-CG cases in one batch, several to a launch, beside a multigrid case."""
+    ps = [CaseParams(nx=64, ny=16, nz=32, Re=200.0, mu_plus=3.0, seed=1, noise=1e-2),
+          CaseParams(nx=33, ny=14, nz=21, Re=150.0, mu_plus=2.0, seed=2, noise=1e-2),
+          CaseParams(nx=64, ny=16, nz=32, Re=300.0, mu_plus=5.0, seed=3, noise=1e-2, ksp_pc="mg"),
+          CaseParams(nx=96, ny=30, nz=50, Re=120.0, mu_plus=2.0, seed=4, noise=1e-2)]
+    prec = ["fp64", "fp64", "fp64", "fp32"]
+
+    def make():
+        cs = [Case(p, precision=q) for p, q in zip(ps, prec)]
+        for c, p in zip(cs, ps):
+            c.load(*make_initial(p))
+        return cs
+
+    alone, batch = make(), make()
+    for c in alone:
+        c.step(3)
+    set_batch_grouped(mode)
+    try:
+        batch_step(batch, 3)
+    finally:
+        set_batch_grouped(1)
+    for a, b in zip(alone, batch):
+        assert a.diag() == b.diag()
+        for f in ("u2", "v2", "w2", "phi2", "pres"):
+            assert np.array_equal(a.field(f), b.field(f))

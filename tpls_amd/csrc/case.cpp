@@ -161,6 +161,14 @@ struct tpls_case {
     double* red_out = nullptr;
     CgState* cg = nullptr;
     CgState* h_cg = nullptr;   // pinned host mirror
+    // the plain CG on the chip (cg_chip.hip): its boxes, device table and
+    // workspace, and the number of the next solve's first reduction
+    bool chip = false;
+    CgChipPlan chip_plan{};
+    CgChipCase chip_h{};         // the table's contents
+    CgChipCase* chip_d = nullptr;
+    void* chip_ws = nullptr;
+    unsigned chip_epoch = 1;
     double* h_out = nullptr;   // pinned host mirror of red_out
     tpls_diag diag{};
     long steps_done = 0;
@@ -480,7 +488,9 @@ size_t tpls_case_bytes(int maxl, int maxm, int maxn, int precision)
     n += p * esz * (3 + 4 + 3 + 4 + 1 + 1);  // cphi, phi2/3/ra/rb, D/sg/ist, fx/fy/fz, mu, ConvPrevPhi
     n += p * esz;                            // pres
     n += pd * rows * (maxn + 1) * 8 * 4;     // pold + CG vectors
-    n += pd * rows * (maxn + 1) * 8 * 2;     // multigrid z and coarse levels (< 1/7 x 2), if enabled
+    // multigrid z and coarse levels (< 1/7 x 2), if enabled; the plain CG's
+    // workspace on the chip is smaller
+    n += pd * rows * (maxn + 1) * 8 * 2;
     return n + (1 << 20);
 }
 
@@ -633,6 +643,13 @@ int tpls_case_create(const tpls_params* prm, int maxl, int maxm, int maxn, tpls_
             }
         }
     }
+    if (!c->use_mg && cg_chip_plan(maxl - 1, maxm - 1, maxn - 1, &c->chip_plan) && cg_chip_fits_device(c->chip_plan)) {
+        const size_t slots = cg_chip_slot_bytes(c->chip_plan), faces = cg_chip_face_bytes(c->chip_plan);
+        if (hipMalloc(&c->chip_ws, slots + faces) != hipSuccess || hipMalloc(&c->chip_d, sizeof(CgChipCase)) != hipSuccess)
+            return bail(fail(TPLS_ERR_NOMEM, "workspace of the pressure solve"));
+        if (hipMemsetAsync(c->chip_ws, 0, slots + faces, c->s) != hipSuccess) return bail(fail(TPLS_ERR_HIP, "memset"));
+        c->chip = true;
+    }
     const long nb = std::max<long>(cg_num_blocks(c->g), (long)REDUCE_BLOCKS);
     if (hipMalloc(&c->red_part, sizeof(double) * 3 * nb) != hipSuccess) return bail(fail(TPLS_ERR_NOMEM, "partials"));
     if (hipMalloc(&c->red_out, sizeof(double) * 8) != hipSuccess) return bail(fail(TPLS_ERR_NOMEM, "outs"));
@@ -658,6 +675,8 @@ int tpls_case_destroy(tpls_case* c)
     hipFree(c->red_part);
     hipFree(c->red_out);
     hipFree(c->cg);
+    hipFree(c->chip_ws);
+    hipFree(c->chip_d);
     hipFree(c->mg_spec);
     hipFree(c->dim_prof);
     if (c->h_cg) hipHostFree(c->h_cg);
@@ -1005,10 +1024,60 @@ int capture(tpls_case* c, hipGraphExec_t* out, F&& fn)
     return rc;
 }
 
+// Whether the case's solve runs as one launch on the chip (cg_chip.hip).  The
+// CG update timed by itself is the streaming kernel.
+bool on_chip(const tpls_case* c) { return c->chip && c->timed != TPLS_TIME_CG_X; }
+
+// The case's entry of an on-chip launch, its table brought up to date (the
+// spacings of a drop-in solve change between calls).
+int chip_entry(tpls_case* c, hipStream_t s, CgChipLaunch* out)
+{
+    const CgChipPlan& p = c->chip_plan;
+    const Phys& ph = c->ph;
+    CgChipCase k;
+    std::memset(&k, 0, sizeof k);  // compared as bytes below
+    k.nx = c->maxl - 1, k.ny = c->g.P, k.nz = c->maxn - 1;
+    // pressure_solver.F90:394-421, as make_op of the streaming kernels
+    k.cz = 1.0 / (ph.dz * ph.dz);
+    k.cx = 1.0 / (ph.dy * ph.dy);
+    k.cy = 1.0 / (ph.dx * ph.dx);
+    k.diag = 2.0 * (1.0 / (ph.dx * ph.dx) + 1.0 / (ph.dy * ph.dy) + 1.0 / (ph.dz * ph.dz));
+    k.gx = p.gx, k.gy = p.gy, k.gz = p.gz, k.bx = p.bx, k.by = p.by, k.bz = p.bz, k.nseg = p.nseg;
+    k.x = c->pold->view<double>();
+    k.r = c->cg_r->view<double>();
+    k.st = c->cg;
+    k.slots = static_cast<unsigned long long*>(c->chip_ws);
+    k.faces = reinterpret_cast<double*>(static_cast<char*>(c->chip_ws) + cg_chip_slot_bytes(p));
+    if (std::memcmp(&k, &c->chip_h, sizeof k) != 0) {
+        // earlier solves of the case have finished: each is waited for
+        c->chip_h = k;
+        LCHK(hipMemcpyAsync(c->chip_d, &c->chip_h, sizeof k, hipMemcpyHostToDevice, s));
+        LCHK(hipStreamSynchronize(s));
+    }
+    *out = {&c->chip_plan, c->chip_d, c->chip_epoch};
+    c->chip_epoch += 2 * unsigned(std::max(1, c->prm.ksp_maxits)) + 2;
+    return TPLS_OK;
+}
+
+// A solve on the chip that waited too long for another block.
+int chip_check(const CgState& st)
+{
+    return st.pad ? fail(TPLS_ERR_HIP, "the pressure solve's blocks waited too long for each other") : int(TPLS_OK);
+}
+
 int ps_enqueue_chunk(tpls_case* c)
 {
     const Grid& g = c->g;
     const bool mg = c->use_mg;
+    if (on_chip(c)) {
+        CgChipLaunch l;
+        RC(chip_entry(c, c->s, &l));
+        LCHK(launch_cg_chip(c->s, {l}));
+        c->ps_launched = std::max(1, c->prm.ksp_maxits);
+        LCHK(hipMemcpyAsync(c->h_cg, c->cg, sizeof(CgState), hipMemcpyDeviceToHost, c->s));
+        LCHK(hipEventRecord(c->ps_ev, c->s));
+        return TPLS_OK;
+    }
     FieldView<double> x = c->pold->view<double>(), r = c->cg_r->view<double>();
     const bool z32 = mg && c->mg.fp32;
     FieldView<double> z = mg && !z32 ? c->cg_z->view<double>() : r;
@@ -1113,6 +1182,7 @@ int ps_poll(tpls_case* c, bool* finished)
         int rc = harvest_events(c);
         if (rc) return rc;
     }
+    RC(chip_check(*c->h_cg));
     if (c->h_cg->done || c->ps_launched >= c->prm.ksp_maxits) {
         c->diag.ksp_its = c->h_cg->its;
         c->diag.ksp_reason = c->h_cg->reason;
@@ -1553,6 +1623,8 @@ int group_for(const std::vector<tpls_case*>& cs, SolveGroup** out)
     std::vector<CgGroupCase> cg;
     std::vector<const CgState*> src;
     for (tpls_case* c : cs) {
+        src.push_back(c->cg);
+        if (on_chip(c)) continue;  // launched apart (launch_cg_chip)
         const bool z32 = c->use_mg && c->mg.fp32;
         CgGroupCase k{};
         k.g = c->g;
@@ -1569,7 +1641,6 @@ int group_for(const std::vector<tpls_case*>& cs, SolveGroup** out)
         k.st = c->cg;
         cg.push_back(k);
         if (c->use_mg) mg.push_back(MgGroupCase{&c->mg, c->g, c->red_part, c->cg});
-        src.push_back(c->cg);
     }
     G->any_mg = !mg.empty();
     if (mg_group_vcycle(G->vc, mg)) return fail(TPLS_ERR_ARG, "a multigrid hierarchy the grouped solve cannot run");
@@ -1655,15 +1726,23 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
         LCHK(hipStreamWaitEvent(G->s, c->ps_ev, 0));
     }
     LCHK(G->hh.run(G->s));
+    std::vector<CgChipLaunch> chip;
+    for (tpls_case* c : cs)
+        if (on_chip(c)) {
+            chip.emplace_back();
+            RC(chip_entry(c, G->s, &chip.back()));
+        }
+    LCHK(launch_cg_chip(G->s, chip));
     LCHK(G->vc.run(G->s));
-    long first = 1, launched = 0, maxits = 1;
+    long first = chip.size() == cs.size() ? 0 : 1, launched = 0, maxits = 1;
     for (tpls_case* c : cs) {
+        if (on_chip(c)) continue;
         first = std::max<long>(first, c->use_mg ? std::max(4, c->last_its) : std::max(8, c->last_its - 2));
         maxits = std::max<long>(maxits, c->prm.ksp_maxits);
     }
     int cur = 0;
     for (long chunk = first;;) {
-        chunk = std::min<long>(chunk, std::max<long>(1, maxits - launched));
+        if (first) chunk = std::min<long>(chunk, std::max<long>(1, maxits - launched));
         for (long q = 0; q < chunk; ++q) {
             LCHK(G->it[cur].run(G->s));
             cur ^= 1;
@@ -1674,8 +1753,10 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
         LCHK(hipEventRecord(G->ev, G->s));
         LCHK(hipEventSynchronize(G->ev));
         bool all = true;
-        for (int q = 0; q < G->n; ++q)
-            if (!G->h_st[q].done && launched < cs[q]->prm.ksp_maxits) all = false;
+        for (int q = 0; q < G->n; ++q) {
+            RC(chip_check(G->h_st[q]));
+            if (!on_chip(cs[q]) && !G->h_st[q].done && launched < cs[q]->prm.ksp_maxits) all = false;
+        }
         if (all) break;
         chunk = G->any_mg ? 2 : 16;
     }

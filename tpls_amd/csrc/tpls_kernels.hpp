@@ -4,6 +4,8 @@
 // domain sx = 1, ex = maxl-1, sy = 1, ey = maxm-1.
 #pragma once
 
+#include <vector>
+
 #include "tpls_dev.hpp"
 
 namespace tpls {
@@ -208,6 +210,42 @@ hipError_t launch_cg_p(hipStream_t s, const Grid& g, const Phys& ph, FieldView<Z
                        CgState* st);
 hipError_t launch_cg_x(hipStream_t s, const Grid& g, const Phys& ph, FieldView<double> p,
                        FieldView<double> x, FieldView<double> r, Reduce red2, CgState* st);
+
+// ---- the plain CG of a grid that fits on the chip, one launch (cg_chip.hip) ----
+constexpr int CG_CHIP_BLOCKS = 256;         // boxes at most: one block per CU
+constexpr size_t CG_CHIP_LDS = 152 * 1024;  // p and its halo
+constexpr int CG_CHIP_MAX = 16;             // cases per launch
+struct CgChipPlan {
+    int cells, threads, nseg, nblk, fstride;
+    int bx, by, bz, gx, gy, gz;  // box extents and counts
+    size_t lds;
+};
+// One case's solve, in device memory.
+struct CgChipCase {
+    int nx, ny, nz;
+    double cx, cy, cz, diag;
+    int gx, gy, gz, bx, by, bz, nseg;
+    FieldView<double> x, r;
+    CgState* st;
+    unsigned long long* slots;  // the reductions' words, cg_chip_slot_bytes
+    double* faces;              // w on the box faces, cg_chip_face_bytes
+};
+struct CgChipArgs {
+    int n;
+    const CgChipCase* c[CG_CHIP_MAX];
+    int b0[CG_CHIP_MAX];
+    unsigned epoch[CG_CHIP_MAX];
+};
+struct CgChipLaunch {
+    const CgChipPlan* plan;
+    const CgChipCase* dev;
+    unsigned epoch;  // the solve's first reduction; it numbers two per iteration
+};
+bool cg_chip_plan(int nx, int ny, int nz, CgChipPlan* out);
+bool cg_chip_fits_device(const CgChipPlan& p);
+size_t cg_chip_slot_bytes(const CgChipPlan& p);
+size_t cg_chip_face_bytes(const CgChipPlan& p);
+hipError_t launch_cg_chip(hipStream_t s, const std::vector<CgChipLaunch>& cases);
 template <typename T>
 hipError_t launch_pres_ghosts(hipStream_t s, const Grid& g, const Phys& ph, FieldView<double> x,
                               FieldView<T> u3, const T* u_inlet, FieldView<T> pres);
