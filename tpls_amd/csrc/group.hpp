@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
+#include <type_traits>
 #include <functional>
 #include <vector>
 
@@ -57,6 +58,10 @@ __device__ __forceinline__ int group_find(const int* starts, int n, int b)
     }
 }
 
+// Ops that copy their arguments themselves (from the table, not a register copy).
+template <class Op>
+struct GroupByRef : std::false_type {};
+
 template <class Op>
 __global__ void __launch_bounds__(Op::THREADS) k_group(const GroupItem<typename Op::Args>* tab, const int* starts,
                                                        int n)
@@ -65,8 +70,13 @@ __global__ void __launch_bounds__(Op::THREADS) k_group(const GroupItem<typename 
     const GroupItem<typename Op::Args>& it = tab[group_find(starts, n, b)];
     const int lb = b - it.start;
     if (lb >= it.gx * it.gy * it.gz) return;
-    const typename Op::Args a = it.a;
-    Op::run(a, Blk{lb % it.gx, (lb / it.gx) % it.gy, lb / (it.gx * it.gy), it.gx});
+    const Blk bk{lb % it.gx, (lb / it.gx) % it.gy, lb / (it.gx * it.gy), it.gx};
+    if constexpr (GroupByRef<Op>::value) {
+        Op::run(it.a, bk);
+    } else {
+        const typename Op::Args a = it.a;
+        Op::run(a, bk);
+    }
 }
 
 // The tables of a sequence of grouped launches, packed into one device

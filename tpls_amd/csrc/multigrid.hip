@@ -649,111 +649,6 @@ __global__ void __launch_bounds__(BX* BY) k_mg_prolong(MgLevelT<XF, BF> f, MgLev
     MgProlong<XF, BF, XC>::run({f, c, st}, blk_here());
 }
 
-// Levels of at most MG1_CELLS cells are visited in one block (k_mg_bottom):
-// on the way down the first pre-smoothing pair and the nu - 1 pairs (red,
-// black) after it, on the way up the prolongation and the nu pairs (black,
-// red).  Each sweep covers the level's column pairs block-stride with
-// mg_pre_cells / mg_smooth_cell / mg_prolong_cells, a barrier between
-// sweeps: every cell computes what k_mg_pre, k_mg_smooth and k_mg_prolong
-// compute (within a colour the updates are order-free).
-constexpr int MG1_T = 1024;
-constexpr long MG1_CELLS = 8192;
-template <typename L>
-static bool mg_one_block(const L& o) { return long(o.nx) * o.ny * o.nz <= MG1_CELLS; }
-
-template <typename X, typename B, typename F>
-__device__ __forceinline__ void mg1_pairs(const MgLevelT<X, B>& o, F&& cell)
-{
-    const int hx = o.nx / 2, n = hx * o.ny * o.nz;
-    for (int q = int(threadIdx.x); q < n; q += MG1_T) {
-        const int r = q / hx;
-        cell(2 * (q % hx) + 1, r % o.ny + 1, r / o.ny + 1);
-    }
-    __syncthreads();
-}
-
-// The visits of one such level, in the block.
-template <typename X, typename B>
-__device__ __forceinline__ void mg1_down(const MgLevelT<X, B>& o, int nu)
-{
-    const FieldView<X> nobc{nullptr, 0, 0};
-    mg1_pairs(o, [&](int i0, int j, int k) { mg_pre_cells(o, nobc, i0, j, k); });
-    for (int q = 1; q < nu; ++q) {
-        mg1_pairs(o, [&](int i0, int j, int k) { mg_smooth_cell(o, 0, i0, j, k); });
-        mg1_pairs(o, [&](int i0, int j, int k) { mg_smooth_cell(o, 1, i0, j, k); });
-    }
-}
-
-template <typename X, typename B, typename XC>
-__device__ __forceinline__ void mg1_up(const MgLevelT<X, B>& o, const MgLevelT<XC, XC>& c, int nu)
-{
-    // the prolongation: one thread per coarse column I and fine (j, k)
-    const int n = c.nx * o.ny * o.nz;
-    for (int q = int(threadIdx.x); q < n; q += MG1_T) {
-        const int r = q / c.nx;
-        mg_prolong_cells(o, c, q % c.nx + 1, r % o.ny + 1, r / o.ny + 1);
-    }
-    __syncthreads();
-    for (int q = 0; q < nu; ++q) {
-        mg1_pairs(o, [&](int i0, int j, int k) { mg_smooth_cell(o, 1, i0, j, k); });
-        mg1_pairs(o, [&](int i0, int j, int k) { mg_smooth_cell(o, 0, i0, j, k); });
-    }
-}
-
-// The residual-restriction f -> c in the block: every fine cell's residual
-// into LDS (r), then each coarse cell's b_c = P^T r / 8 with k_mg_rr's sums
-// (along x, then y, then z, each over the candidates q = 0..3 with nonzero
-// weight, in order), so the coarse values are k_mg_rr's bit for bit.
-template <typename X>
-__device__ __forceinline__ void mg1_rr(const MgLevelT<X, X>& f, const MgLevelT<X, X>& c, X* r)
-{
-    using C = X;
-    const int nf = f.nx * f.ny * f.nz;
-    for (int q = int(threadIdx.x); q < nf; q += MG1_T) {
-        const int i = q % f.nx + 1, rr = q / f.nx, j = rr % f.ny + 1, k = rr / f.ny + 1;
-        const int jm = j == 1 ? f.ny : j - 1, jp = j == f.ny ? 1 : j + 1;
-        const C xc = f.x(i, j, k);
-        const C zm = k > 1 ? C(f.x(i, j, k - 1)) : C(0);
-        const C zp = k < f.nz ? C(f.x(i, j, k + 1)) : C(0);
-        const C xm = i > 1 ? C(f.x(i - 1, j, k)) : C(0);
-        const C xp = i < f.nx ? C(f.x(i + 1, j, k)) : C(0);
-        const C ym = f.x(i, jm, k), yp = f.x(i, jp, k);
-        const C nsum = C(f.cz) * (zm + zp) + C(f.cx) * (xm + xp) + C(f.cy) * (ym + yp);
-        r[q] = C(f.b(i, j, k)) - (mg_deff<C>(f, i, k) * xc - nsum);
-    }
-    __syncthreads();
-    const int nc = c.nx * c.ny * c.nz;
-    for (int q = int(threadIdx.x); q < nc; q += MG1_T) {
-        const int I = q % c.nx + 1, rr = q / c.nx, J = rr % c.ny + 1, K = rr / c.ny + 1;
-        C wi[4], wj[4], wk[4];
-        mg_rweights_q(I, c.nx, f.nx, false, wi);
-        mg_rweights_q(J, c.ny, f.ny, true, wj);
-        mg_rweights_q(K, c.nz, f.nz, false, wk);
-        C sk = 0;
-#pragma unroll
-        for (int qz = 0; qz < 4; ++qz) {
-            if (wk[qz] == C(0)) continue;
-            const int fk = 2 * K - 2 + qz;
-            C sj = 0;
-#pragma unroll
-            for (int qy = 0; qy < 4; ++qy) {
-                if (wj[qy] == C(0)) continue;
-                int fj = 2 * J - 2 + qy;
-                if (fj < 1) fj += f.ny;
-                if (fj > f.ny) fj -= f.ny;
-                C si = 0;
-#pragma unroll
-                for (int qx = 0; qx < 4; ++qx)
-                    if (wi[qx] != C(0)) si += wi[qx] * r[(2 * I - 2 + qx - 1) + f.nx * ((fj - 1) + f.ny * (fk - 1))];
-                sj += wj[qy] * si;
-            }
-            sk += wk[qz] * sj;
-        }
-        c.b(I, J, K) = C(0.125) * sk;
-    }
-    __syncthreads();
-}
-
 // Coarsest level: one block, a single wavefront for up to 64 cells (its
 // barriers cost next to nothing), else 256 threads; x and b live in LDS
 // (n <= MG_COARSE_MAX).  Each thread's cells, their colours and diagonals are
@@ -772,15 +667,13 @@ struct MgCoarse {
     static __device__ __forceinline__ void run(const Args& a, const Blk&);
 };
 
-template <typename X>
-__device__ __forceinline__ void MgCoarse<X>::run(const Args& a, const Blk&)
+// get(i, j, k) reads the right-hand side, put(i, j, k, v) takes the solution;
+// sx, sb: LDS of the level's cells each, apart from what get reads.
+template <typename C, typename L, typename Get, typename Put>
+__device__ __forceinline__ void mg_coarse_solve(const L& o, C* sx, C* sb, Get&& get, Put&& put)
 {
-    using C = X;
-    const MgLevelT<X, X>& o = a.o;
-    if (a.st->done) return;
-    __shared__ C sx[MG_COARSE_MAX], sb[MG_COARSE_MAX];
     __shared__ C mean;
-    const int tid = threadIdx.x, nt = blockDim.x;
+    const int tid = threadIdx.x, nt = min(int(blockDim.x), MGC_T);
     const int n = o.nx * o.ny * o.nz;
     int ci[MGC_CPT], cj[MGC_CPT], ck[MGC_CPT], col[MGC_CPT];
     C cd[MGC_CPT];
@@ -791,14 +684,14 @@ __device__ __forceinline__ void MgCoarse<X>::run(const Args& a, const Blk&)
         const int r = q / o.nx;
         cj[c] = r % o.ny + 1;
         ck[c] = r / o.ny + 1;
-        col[c] = tid + c * nt < n ? (ci[c] + cj[c] + ck[c]) & 1 : 2;  // 2: no cell
+        col[c] = tid < nt && tid + c * nt < n ? (ci[c] + cj[c] + ck[c]) & 1 : 2;  // 2: no cell
         cd[c] = mg_deff<C>(o, ci[c], ck[c]);
     }
 #pragma unroll
     for (int c = 0; c < MGC_CPT; ++c)
         if (col[c] != 2) {
             const int q = tid + c * nt;
-            sb[q] = o.b(ci[c], cj[c], ck[c]);
+            sb[q] = get(ci[c], cj[c], ck[c]);
             sx[q] = 0;
         }
     __syncthreads();
@@ -809,7 +702,7 @@ __device__ __forceinline__ void MgCoarse<X>::run(const Args& a, const Blk&)
     }
     __syncthreads();
     const C mb = mean;
-    for (int q = tid; q < n; q += nt) sb[q] = sb[q] - mb;
+    for (int q = tid; q < n; q += blockDim.x) sb[q] = sb[q] - mb;
     __syncthreads();
     const int nmax = max(o.nx, max(o.ny, o.nz));
     const int sweeps = 20 + nmax * nmax / 2;
@@ -835,7 +728,17 @@ __device__ __forceinline__ void MgCoarse<X>::run(const Args& a, const Blk&)
     const C mx = mean;
 #pragma unroll
     for (int c = 0; c < MGC_CPT; ++c)
-        if (col[c] != 2) o.x(ci[c], cj[c], ck[c]) = sx[tid + c * nt] - mx;
+        if (col[c] != 2) put(ci[c], cj[c], ck[c], sx[tid + c * nt] - mx);
+}
+
+template <typename X>
+__device__ __forceinline__ void MgCoarse<X>::run(const Args& a, const Blk&)
+{
+    const MgLevelT<X, X>& o = a.o;
+    if (a.st->done) return;
+    __shared__ X sx[MG_COARSE_MAX], sb[MG_COARSE_MAX];
+    mg_coarse_solve(o, sx, sb, [&](int i, int j, int k) { return o.b(i, j, k); },
+                    [&](int i, int j, int k, X v) { o.x(i, j, k) = v; });
 }
 
 template <typename X>
@@ -848,6 +751,83 @@ __global__ void __launch_bounds__(MGC_T) k_mg_coarse(MgLevelT<X, X> o, const CgS
 // storage: b into LDS, b^ = Qz^T Qy^T Qx^T b (one pass per direction, each
 // output summed over its line in index order), b^ / lambda with the constant
 // mode dropped, then z = Qx Qy Qz b^.  tab: mg_spectral_tables.
+//
+// 1024 threads, and the tables in LDS where they are small (up to MGS_TAB
+// values): with 256 threads reading them from the caches a solve of 22x6x10
+// or 24x6x12 cells took 29 us, 10 and 13 us now.  The six passes are one loop
+// body: code that runs once per launch costs an instruction-cache miss per
+// line, more than its arithmetic.
+constexpr int MGS_T = 1024, MGS_TAB = 1024;
+
+// s0, s1: LDS of the level's cells each; st: LDS of MGS_TAB values.
+template <typename L, typename Get, typename Put>
+__device__ __forceinline__ void mg_spec_solve(const L& o, const double* tab, double* s0, double* s1, double* st,
+                                              Get&& get, Put&& put)
+{
+    const int tid = threadIdx.x, nt = blockDim.x;
+    const int nx = o.nx, ny = o.ny, nz = o.nz, n = nx * ny * nz;
+    const int ntab = nx * nx + ny * ny + nz * nz + nx + ny + nz;
+    if (ntab <= MGS_TAB)
+        for (int q = tid; q < ntab; q += nt) st[q] = tab[q];
+    const double shift = o.diag - 2.0 * (o.cx + o.cy + o.cz);
+    // (a thread's first element's coordinates are worked out once)
+    const int r0 = tid / nx, k0 = r0 / ny, j0 = r0 - k0 * ny, i0 = tid - r0 * nx;
+    auto each = [&](auto&& f) {
+        int i = i0, j = j0, k = k0;
+#pragma unroll 1
+        for (int q = tid; q < n;) {
+            f(q, i, j, k);
+            q += nt;
+            if (q >= n) break;
+            const int r = q / nx;
+            k = r / ny, j = r - k * ny, i = q - r * nx;
+        }
+        __syncthreads();
+    };
+    each([&](int q, int i, int j, int k) { s0[q] = double(get(i + 1, j + 1, k + 1)); });
+    auto solve = [&](const double* Qx) {
+        const double* Qy = Qx + nx * nx;
+        const double* Qz = Qy + ny * ny;
+        const double* ev = Qz + nz * nz;
+        const double *in = s0, *lx = ev, *ly = ev + nx, *lz = ev + nx + ny;
+        double* out = s1;
+#pragma unroll 1
+        for (int d6 = 0; d6 < 6; ++d6) {
+            const bool fwd = d6 < 3;
+            const int d = fwd ? d6 : 5 - d6;
+            const int nd = d == 0 ? nx : (d == 1 ? ny : nz), stride = d == 0 ? 1 : (d == 1 ? nx : nx * ny);
+            const double* Q = d == 0 ? Qx : (d == 1 ? Qy : Qz);
+            each([&](int q, int i, int j, int k) {
+                const int c = d == 0 ? i : (d == 1 ? j : k);
+                const double* qp = fwd ? Q + c : Q + c * nd;
+                const double* ip = in + (q - c * stride);
+                const int qs = fwd ? nd : 1;
+                double acc = 0.0;
+                int m = 0;
+#pragma unroll 1
+                for (; m + 4 <= nd; m += 4) {
+                    double a[4], b[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) a[u] = qp[(m + u) * qs], b[u] = ip[(m + u) * stride];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) acc += a[u] * b[u];
+                }
+#pragma unroll 1
+                for (; m < nd; ++m) acc += qp[m * qs] * ip[m * stride];
+                if (d6 == 2) acc = q == 0 ? 0.0 : acc / (shift + o.cx * lx[i] + o.cy * ly[j] + o.cz * lz[k]);
+                out[q] = acc;
+            });
+            double* const t = const_cast<double*>(in);
+            in = out;
+            out = t;
+        }
+    };
+    // (the LDS and the memory tables by separate code, for their own loads)
+    if (ntab <= MGS_TAB) solve(st);
+    else solve(tab);
+    each([&](int q, int i, int j, int k) { put(i + 1, j + 1, k + 1, s0[q]); });
+}
+
 template <typename X, typename B>
 struct MgSpec {
     struct Args {
@@ -855,95 +835,338 @@ struct MgSpec {
         const double* tab;
         const CgState* st;
     };
-    static constexpr int THREADS = MGC_T;
-    static dim3 block() { return dim3(MGC_T); }
-    static __device__ __forceinline__ void run(const Args& a, const Blk&);
+    static constexpr int THREADS = MGS_T;
+    static dim3 block() { return dim3(MGS_T); }
+    static __device__ __forceinline__ void run(const Args& a, const Blk&)
+    {
+        const MgLevelT<X, B>& o = a.o;
+        if (a.st->done) return;
+        __shared__ double s0[MG_COARSE_MAX], s1[MG_COARSE_MAX], tb[MGS_TAB];
+        mg_spec_solve(o, a.tab, s0, s1, tb, [&](int i, int j, int k) { return o.b(i, j, k); },
+                      [&](int i, int j, int k, double v) { o.x(i, j, k) = X(v); });
+    }
 };
 
 template <typename X, typename B>
-__device__ __forceinline__ void MgSpec<X, B>::run(const Args& a, const Blk&)
-{
-    const MgLevelT<X, B>& o = a.o;
-    const double* tab = a.tab;
-    if (a.st->done) return;
-    __shared__ double s0[MG_COARSE_MAX], s1[MG_COARSE_MAX];
-    const int tid = threadIdx.x, nt = blockDim.x;
-    const int nx = o.nx, ny = o.ny, nz = o.nz, n = nx * ny * nz;
-    const double* Qx = tab;
-    const double* Qy = Qx + nx * nx;
-    const double* Qz = Qy + ny * ny;
-    const double* lx = Qz + nz * nz;
-    const double* ly = lx + nx;
-    const double* lz = ly + ny;
-    for (int q = tid; q < n; q += nt) {
-        const int r = q / nx;
-        s0[q] = double(o.b(q % nx + 1, r % ny + 1, r / ny + 1));
-    }
-    __syncthreads();
-    // one direction: out = Q^T in (fwd) or Q in along direction d
-    auto pass = [&](const double* in, double* out, int d, bool fwd) {
-        const int nd = d == 0 ? nx : (d == 1 ? ny : nz);
-        const int stride = d == 0 ? 1 : (d == 1 ? nx : nx * ny);
-        const double* Q = d == 0 ? Qx : (d == 1 ? Qy : Qz);
-        for (int q = tid; q < n; q += nt) {
-            const int c = (q / stride) % nd, base = q - c * stride;
-            double acc = 0.0;
-            for (int m = 0; m < nd; ++m) acc += (fwd ? Q[m * nd + c] : Q[c * nd + m]) * in[base + m * stride];
-            out[q] = acc;
-        }
-        __syncthreads();
-    };
-    pass(s0, s1, 0, true);
-    pass(s1, s0, 1, true);
-    pass(s0, s1, 2, true);
-    const double shift = o.diag - 2.0 * (o.cx + o.cy + o.cz);
-    for (int q = tid; q < n; q += nt) {
-        const int r = q / nx;
-        const double ev = shift + o.cx * lx[q % nx] + o.cy * ly[r % ny] + o.cz * lz[r / ny];
-        s1[q] = q == 0 ? 0.0 : s1[q] / ev;
-    }
-    __syncthreads();
-    pass(s1, s0, 2, false);
-    pass(s0, s1, 1, false);
-    pass(s1, s0, 0, false);
-    for (int q = tid; q < n; q += nt) {
-        const int r = q / nx;
-        o.x(q % nx + 1, r % ny + 1, r / ny + 1) = X(s0[q]);
-    }
-}
-
-template <typename X, typename B>
-__global__ void __launch_bounds__(MGC_T) k_mg_spec(MgLevelT<X, B> o, const double* tab, const CgState* st)
+__global__ void __launch_bounds__(MGS_T) k_mg_spec(MgLevelT<X, B> o, const double* tab, const CgState* st)
 {
     MgSpec<X, B>::run({o, tab, st}, blk_here());
 }
+static int spec_threads(long cells) { return int(std::min<long>(MGS_T, (cells + 63) / 64 * 64)); }
 
-// The bottom of the V-cycle in one block: levels L[0] .. L[n-2] (each of at
-// most MG1_CELLS cells) down (mg1_down, mg1_rr) and up (mg1_up) as the
-// multi-block kernels would run them, and the coarsest level L[n-1] as
-// k_mg_spec (tab set) or k_mg_coarse: one launch instead of about
-// (2 nu + 1 + 2 nu + 1) (n - 1) + 1.
+// The bottom of the V-cycle in one block: levels L[0] .. L[n-2] down and up
+// and the coarsest level L[n-1] as k_mg_spec (tab set) or k_mg_coarse, with
+// every level's x and right-hand side, the residual being restricted and the
+// coordinates of every pair of cells in LDS.  A level is visited as the multi-block
+// kernels visit it: on the way down the nu pairs (red, black) from x = 0, on
+// the way up the prolongation and the nu pairs (black, red), a barrier between
+// sweeps; every cell computes what k_mg_pre, k_mg_smooth, k_mg_rr and
+// k_mg_prolong compute (within a colour the updates are order-free).
+//
+// One launch instead of about (4 nu + 2) (n - 1) + 1.  With the vectors in
+// memory each of the about 28 passes waited for the L2: 48 us for levels of
+// 4096, 512 and 64 cells in FP64, 24 us now.  What is left is the
+// first level's sweeps (one CU's FP64 rate) and, in every pass, the latency
+// of LDS and a barrier.  All levels run the same code, loops not unrolled: a
+// pass unrolled per level spent more on instruction-cache misses than on
+// arithmetic (8,800 cycles for a restriction).
+constexpr int MG1_T = 1024;
 constexpr int MG1_MAXLEV = 6;
+constexpr int MG1_LDS = 152 * 1024;
+
+// n / d with r = 1/d: FP64 the correctly rounded quotient (Markstein: the
+// product with the correctly rounded reciprocal, corrected once by its
+// residual), in three operations for the division's fifteen; FP32 as sdiv.
+template <typename C>
+struct Mg1Diag {
+    C d, r;
+};
+__device__ __forceinline__ double mg1_quot(double n, const Mg1Diag<double>& q)
+{
+    const double t = n * q.r;
+    return __builtin_fma(__builtin_fma(-q.d, t, n), q.r, t);
+}
+__device__ __forceinline__ float mg1_quot(float n, const Mg1Diag<float>& q) { return n * q.r; }
+
+// A value that is the same in every lane, in a scalar register.
+__device__ __forceinline__ int mg1_uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// Lane q of each quad's value, in its four lanes.
+template <int Q>
+__device__ __forceinline__ float mg1_quad(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), Q * 0x55, 0xf, 0xf, true));
+}
+template <int Q>
+__device__ __forceinline__ double mg1_quad(double v)
+{
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), Q * 0x55, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), Q * 0x55, 0xf, 0xf, true));
+}
+
 template <typename X>
-struct MgBottom {
+struct MgBottomArgs {
     MgLevelT<X, X> L[MG1_MAXLEV];
     int n, nu;
+    int ox[MG1_MAXLEV], ob[MG1_MAXLEV], orr;  // places of x, b and r in LDS
+    int op[MG1_MAXLEV];                       // and of the pairs' coordinates
+    unsigned mx[MG1_MAXLEV], mh[MG1_MAXLEV], my[MG1_MAXLEV];  // 2^32 / nx, / (nx/2) and / ny, rounded up
+    const double* tab;
+    const CgState* st;
 };
+template <typename X>
+struct MgBottom {
+    using Args = MgBottomArgs<X>;
+    static constexpr int THREADS = MG1_T;
+    static dim3 block() { return dim3(MG1_T); }
+    static __device__ __forceinline__ void run(const Args& a, const Blk&);
+};
+template <typename X>
+struct GroupByRef<MgBottom<X>> : std::true_type {};
+
+// The levels lev[lb] .. lev[last]: false if one block cannot take them.
+template <typename X>
+static bool mg_bottom_args(const MgLevelT<X, X>* lev, int lb, int last, int nu, const double* tab, const CgState* st,
+                           MgBottomArgs<X>* out)
+{
+    MgBottomArgs<X> a{};
+    a.n = last - lb + 1;
+    if (a.n < 2 || a.n > MG1_MAXLEV) return false;
+    a.nu = nu;
+    a.tab = tab;
+    a.st = st;
+    auto cells = [&](int l) { return long(lev[l].nx) * lev[l].ny * lev[l].nz; };
+    auto magic = [](int d) { return unsigned(((1ULL << 32) + d - 1) / d); };
+    long at = 0, pairs = 0;
+    for (int l = lb; l <= last; ++l) {
+        const MgLevelT<X, X>& o = lev[l];
+        a.L[l - lb] = o;
+        if (l < last) {
+            if (o.nx > 1023 || o.ny > 1023 || o.nz > 1023) return false;
+            a.mh[l - lb] = magic(o.nx / 2);
+            a.op[l - lb] = int(pairs);
+            pairs += cells(l) / 2;
+        }
+        a.mx[l - lb] = magic(o.nx);
+        a.my[l - lb] = magic(o.ny);
+        a.ox[l - lb] = int(at);
+        at += cells(l);
+        a.ob[l - lb] = int(at);
+        at += cells(l);
+    }
+    at = (at + 1) / 2 * 2;
+    a.orr = int(at);
+    // r of the first level, or the coarsest solve's two vectors and tables
+    const long r = std::max<long>((cells(lb) * long(sizeof(X)) + 7) / 8 * 8, (2 * cells(last) + MGS_TAB) * 8);
+    const long place = at * long(sizeof(X)) + r;
+    for (int l = 0; l + 1 < a.n; ++l) a.op[l] += int(place / 8);
+    if (place + pairs * 8 > MG1_LDS) return false;
+    *out = a;
+    return true;
+}
 
 template <typename X>
-__global__ void __launch_bounds__(MG1_T) k_mg_bottom(MgBottom<X> a, const double* tab, const CgState* st)
+__device__ __forceinline__ void MgBottom<X>::run(const Args& args, const Blk&)
 {
-    if (st->done) return;
-    __shared__ X r[MG1_CELLS];
-    const int n = a.n;
-    for (int l = 0; l + 1 < n; ++l) {
-        mg1_down(a.L[l], a.nu);
-        mg1_rr(a.L[l], a.L[l + 1], r);
-    }
-    if (tab) MgSpec<X, X>::run({a.L[n - 1], tab, st}, Blk{0, 0, 0, 1});
-    else MgCoarse<X>::run({a.L[n - 1], st}, Blk{0, 0, 0, 1});
+    using C = X;
+    if (args.st->done) return;
+    // the levels are indexed at run time: from LDS, not from registers
+    __shared__ Args a;
+    __shared__ double raw[MG1_LDS / 8];
+    // a level's diagonals by which ends of z and x the cell is at, in mg_deff's
+    // order of subtractions
+    __shared__ Mg1Diag<C> dg[MG1_MAXLEV][16];
+    const int tid = int(threadIdx.x);
+    for (int q = tid; q < int(sizeof(Args) / 4); q += MG1_T)
+        reinterpret_cast<int*>(&a)[q] = reinterpret_cast<const int*>(&args)[q];
     __syncthreads();
-    for (int l = n - 2; l >= 0; --l) mg1_up(a.L[l], a.L[l + 1], a.nu);
+    C* const lds = reinterpret_cast<C*>(raw);
+    C* const r = lds + a.orr;
+    const int n = a.n, nu = a.nu;
+    if (tid < 16 * (n - 1)) {
+        const MgLevelT<X, X>& o = a.L[tid / 16];
+        const int f = tid % 16;
+        C v = C(o.diag);
+        if (f & 1) v = v - C(o.cz);
+        if (f & 2) v = v - C(o.cz);
+        if (f & 4) v = v - C(o.cx);
+        if (f & 8) v = v - C(o.cx);
+        dg[tid / 16][f] = {v, recip(v)};
+    }
+    // The pairs of cells along x of every level but the last: coordinates
+    // (pair, j - 1, k - 1 in 10 bits each), and which ends of the level they
+    // are at.  q * d < 2^32 for every quotient, so the products with 2^32 / d
+    // are exact.
+    enum { ZLO = 1, ZHI = 2, XLO = 4, XHI = 8, YLO = 16, YHI = 32, ODD = 64 };
+    struct Pr {
+        int e, c, f;  // the first cell's place in LDS, coordinates, ends
+        __device__ __forceinline__ int i0() const { return 2 * (c & 1023) + 1; }
+        __device__ __forceinline__ int j() const { return ((c >> 10) & 1023) + 1; }
+        __device__ __forceinline__ int k() const { return (c >> 20) + 1; }
+    };
+    int2* const place = reinterpret_cast<int2*>(raw);
+    for (int l = 0; l + 1 < n; ++l) {
+        const int hx = mg1_uni(a.L[l].nx) / 2, ny = mg1_uni(a.L[l].ny), nz = mg1_uni(a.L[l].nz), m = hx * ny * nz;
+        const unsigned mh = unsigned(mg1_uni(int(a.mh[l]))), my = unsigned(mg1_uni(int(a.my[l])));
+#pragma unroll 1
+        for (int q = tid; q < m; q += MG1_T) {
+            const int row = int(__umulhi(unsigned(q), mh)), k = int(__umulhi(unsigned(row), my));
+            const int i = q - row * hx, j = row - k * ny;
+            const int ends = (k == 0 ? ZLO : 0) | (k == nz - 1 ? ZHI : 0) | (i == 0 ? XLO : 0) | (i == hx - 1 ? XHI : 0) |
+                             (j == 0 ? YLO : 0) | (j == ny - 1 ? YHI : 0) | ((j + k) & 1 ? 0 : ODD);
+            const Pr p{2 * q, i | j << 10 | k << 20, ends};
+            place[a.op[l] + q] = make_int2(p.c, ends);
+            // x to zero, the first right-hand side into LDS
+            lds[a.ox[l] + 2 * q] = lds[a.ox[l] + 2 * q + 1] = C(0);
+            if (l > 0) continue;
+            const C* b = &a.L[0].b(p.i0(), p.j(), p.k());
+            lds[a.ob[0] + 2 * q] = b[0], lds[a.ob[0] + 2 * q + 1] = b[1];
+        }
+    }
+    __syncthreads();
+    // fn for every pair of level l, then a barrier
+    auto pairs = [&](int l, auto&& fn) {
+        const int m = mg1_uni(a.L[l].nx) / 2 * mg1_uni(a.L[l].ny) * mg1_uni(a.L[l].nz);
+        const int2* const pl = place + mg1_uni(a.op[l]);
+#pragma unroll 1
+        for (int q = tid; q < m; q += MG1_T) {
+            const int2 v = pl[q];
+            fn(Pr{2 * q, v.x, v.y});
+        }
+        __syncthreads();
+    };
+    // the level of each visit: 0 .. n-2 on the way down, n-2 .. 0 up
+#pragma unroll 1
+    for (int visit = 0; visit < 2 * (n - 1); ++visit) {
+        const bool dn = visit < n - 1;
+        const int l = dn ? visit : 2 * (n - 1) - 1 - visit;
+        MgLevelT<X, X> f = a.L[l], c = a.L[l + 1];
+        f.nx = mg1_uni(f.nx), f.ny = mg1_uni(f.ny), f.nz = mg1_uni(f.nz);
+        c.nx = mg1_uni(c.nx), c.ny = mg1_uni(c.ny), c.nz = mg1_uni(c.nz);
+        const int sy = f.nx, sz = f.nx * f.ny;
+        C* const x = lds + a.ox[l];
+        const C* const bl = lds + a.ob[l];
+        // sum of c * neighbour of cell h of the pair (mg_nsum), and its diagonal
+        auto nsum = [&](const Pr& p, int h) {
+            const int e = p.e + h;
+            const bool zlo = p.f & ZLO, zhi = p.f & ZHI, xlo = h == 0 && (p.f & XLO), xhi = h == 1 && (p.f & XHI);
+            const C zm = x[zlo ? e : e - sz], zp = x[zhi ? e : e + sz], xm = x[xlo ? e : e - 1], xp = x[xhi ? e : e + 1];
+            const C ym = x[p.f & YLO ? e + sz - sy : e - sy], yp = x[p.f & YHI ? e - sz + sy : e + sy];
+            return C(f.cz) * ((zlo ? C(0) : zm) + (zhi ? C(0) : zp)) + C(f.cx) * ((xlo ? C(0) : xm) + (xhi ? C(0) : xp)) +
+                   C(f.cy) * (ym + yp);
+        };
+        const Mg1Diag<C>* const dl = dg[l];
+        auto diag = [&](const Pr& p, int h) { return dl[p.f & (h ? ZLO | ZHI | XHI : ZLO | ZHI | XLO)]; };
+        if (!dn) {
+            // x += P e_c with mg_prolong_cells' sums
+            const C* xc = lds + a.ox[l + 1];
+            auto ec = [&](int I, int J, int K) { return xc[(I - 1) + c.nx * ((J - 1) + c.ny * (K - 1))]; };
+            const C q3 = C(0.75), q1 = C(0.25);
+            pairs(l, [&](const Pr& p) {
+                const int e = p.e, i0 = p.i0(), j = p.j(), k = p.k(), I = (i0 + 1) / 2, J = (j + 1) / 2, K = (k + 1) / 2;
+                const int Jn = mg_nbr(j, c.ny, true), Kn = mg_nbr(k, c.nz, false);
+                C b[3];  // columns I, and the neighbours of the odd and the even cell
+#pragma unroll
+                for (int h = 0; h < 3; ++h) {
+                    const int In = h == 0 ? I : mg_nbr(i0 + h - 1, c.nx, false);
+                    const C a0 = q3 * ec(In, J, K) + q1 * ec(In, J, Kn);
+                    const C a1 = q3 * ec(In, Jn, K) + q1 * ec(In, Jn, Kn);
+                    b[h] = q3 * a0 + q1 * a1;
+                }
+                x[e] = x[e] + (q3 * b[0] + q1 * b[1]);
+                x[e + 1] = x[e + 1] + (q3 * b[0] + q1 * b[2]);
+            });
+        }
+#pragma unroll 1
+        for (int s = 0; s < 2 * nu; ++s) {
+            const int colour = (s & 1) ^ (dn ? 0 : 1);
+            pairs(l, [&](const Pr& p) {
+                const int h = (p.f & ODD ? 1 : 0) == colour ? 0 : 1;
+                x[p.e + h] = mg1_quot(bl[p.e + h] + nsum(p, h), diag(p, h));
+            });
+        }
+        if (!dn) continue;
+        pairs(l, [&](const Pr& p) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) r[p.e + h] = bl[p.e + h] - (diag(p, h).d * x[p.e + h] - nsum(p, h));
+        });
+        // the coarse right-hand side P^T r / 8 with k_mg_rr's sums (along x,
+        // then y, then z, over the candidates q = 0..3), the four z planes of a
+        // cell by the four lanes of a quad; a candidate of weight 0 adds 0,
+        // with no branch, so that a plane's 16 loads are in flight together
+        const int nc = c.nx * c.ny * c.nz;
+        C* const bc = lds + a.ob[l + 1];
+        const unsigned mxc = unsigned(mg1_uni(int(a.mx[l + 1]))), myc = unsigned(mg1_uni(int(a.my[l + 1])));
+        // (4 nc is a multiple of 4: a quad's lanes leave the loop together)
+#pragma unroll 1
+        for (int t4 = tid; t4 < 4 * nc; t4 += MG1_T) {
+            const int q = t4 >> 2, qz = t4 & 3;
+            const int row = int(__umulhi(unsigned(q), mxc)), K = int(__umulhi(unsigned(row), myc)) + 1;
+            const int I = q - row * c.nx + 1, J = row - (K - 1) * c.ny + 1;
+            // mg_rweights_q along x; along y (periodic) 1/4, 3/4, 3/4, 1/4
+            const C wi[4] = {C(I > 1 ? 0.25 : 0), C(I > 1 ? 0.75 : 1), C(I < c.nx ? 0.75 : 1), C(I < c.nx ? 0.25 : 0)};
+            const C wj[4] = {C(0.25), C(0.75), C(0.75), C(0.25)};
+            int xo[4], yo[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                xo[u] = min(max(2 * I - 3 + u, 0), f.nx - 1);
+                const int fj = 2 * J - 2 + u;
+                yo[u] = sy * (fj < 1 ? f.ny - 1 : (fj > f.ny ? 0 : fj - 1));
+            }
+            const int fk = 2 * K - 2 + qz, zo = sz * (min(max(fk, 1), f.nz) - 1);
+            C v[4][4];
+#pragma unroll
+            for (int qy = 0; qy < 4; ++qy)
+#pragma unroll
+                for (int qx = 0; qx < 4; ++qx) v[qy][qx] = r[zo + yo[qy] + xo[qx]];
+            const C wk = qz == 1 ? C(K > 1 ? 0.75 : 1) : (qz == 2 ? C(K < c.nz ? 0.75 : 1) : C(0.25));
+            C sj = 0;
+#pragma unroll
+            for (int qy = 0; qy < 4; ++qy) {
+                C si = 0;
+#pragma unroll
+                for (int qx = 0; qx < 4; ++qx) si += wi[qx] != C(0) ? wi[qx] * v[qy][qx] : C(0);
+                sj += wj[qy] * si;
+            }
+            const C tz = fk < 1 || fk > f.nz ? C(0) : wk * sj;
+            const C sk = ((mg1_quad<0>(tz) + mg1_quad<1>(tz)) + mg1_quad<2>(tz)) + mg1_quad<3>(tz);
+            if (qz == 0) bc[q] = C(0.125) * sk;
+        }
+        __syncthreads();
+        if (l < n - 2) continue;
+        // the coarsest level
+        const C* const b = lds + a.ob[n - 1];
+        C* const xc = lds + a.ox[n - 1];
+        auto at = [&](int i, int j, int k) { return (i - 1) + c.nx * ((j - 1) + c.ny * (k - 1)); };
+        auto get = [&](int i, int j, int k) { return b[at(i, j, k)]; };
+        if (a.tab) {
+            double* s = reinterpret_cast<double*>(r);
+            mg_spec_solve(c, a.tab, s, s + nc, s + 2 * nc, get,
+                          [&](int i, int j, int k, double v) { xc[at(i, j, k)] = C(v); });
+        } else {
+            mg_coarse_solve(c, r, r + nc, get, [&](int i, int j, int k, C v) { xc[at(i, j, k)] = v; });
+            __syncthreads();
+        }
+    }
+    pairs(0, [&](const Pr& p) {
+        C* const xp = &a.L[0].x(p.i0(), p.j(), p.k());
+        xp[0] = lds[p.e], xp[1] = lds[p.e + 1];
+    });
+}
+
+template <typename X>
+__global__ void __launch_bounds__(MG1_T) k_mg_bottom(MgBottomArgs<X> a)
+{
+    MgBottom<X>::run(a, blk_here());
+}
+
+// The first of the levels that run in one block, or last for none of them.
+template <typename X>
+static int mg_bottom_first(const MgLevelT<X, X>* lev, int last, int nu, const double* tab, const CgState* st,
+                           MgBottomArgs<X>* out)
+{
+    for (int lb = std::max(1, last + 1 - MG1_MAXLEV); lb < last; ++lb)
+        if (mg_bottom_args<X>(lev, lb, last, nu, tab, st, out)) return lb;
+    return last;
 }
 
 // Final red sweep on the finest level with the partials of z.r (r = b) and
@@ -1163,12 +1386,10 @@ static hipError_t vcycle(hipStream_t s, const Grid& g, const MgLevelT<X, double>
     // in the level's own vector, which level 0's prolongation reads.
     const bool pairs1 = last > 1 && x21.p;
     FieldView<X> cur1 = lev[1].x;
-    // levels lb .. last, each of at most MG1_CELLS cells (at least one of
-    // them smoothed), run as one single-block launch (k_mg_bottom)
-    int lb = last;
-    while (lb > 1 && mg_one_block(lev[lb - 1])) --lb;
-    const bool bottom = last > 1 && lb < last && last - lb + 1 <= MG1_MAXLEV;
-    const int lmid = bottom ? lb : last;
+    // levels lmid .. last (at least one of them smoothed) as one launch, or
+    // lmid = last and the coarsest solve by itself
+    MgBottomArgs<X> mb;
+    const int lmid = last > 1 ? mg_bottom_first<X>(lev, last, nu, spec, st, &mb) : last;
     for (int l = 1; l < lmid; ++l) {
         if (l == 1 && pairs1) {
             MgLevelT<X, X> o = lev[1];
@@ -1179,17 +1400,13 @@ static hipError_t vcycle(hipStream_t s, const Grid& g, const MgLevelT<X, double>
             down(lev[l], lev[l + 1]);
         }
     }
-    if (bottom) {
-        MgBottom<X> mb{};
-        for (int l = lb; l <= last; ++l) mb.L[l - lb] = lev[l];
-        mb.n = last - lb + 1;
-        mb.nu = nu;
-        hipLaunchKernelGGL((k_mg_bottom<X>), dim3(1), dim3(MG1_T), 0, s, mb, spec, st);
+    if (lmid < last) {
+        hipLaunchKernelGGL((k_mg_bottom<X>), dim3(1), dim3(MG1_T), 0, s, mb);
     } else if (last > 0) {
         const MgLevelT<X, X>& c = lev[last];
         const long nc = long(c.nx) * c.ny * c.nz;
         if (spec)
-            hipLaunchKernelGGL((k_mg_spec<X, X>), dim3(1), dim3(nc <= 64 ? 64 : MGC_T), 0, s, c, spec, st);
+            hipLaunchKernelGGL((k_mg_spec<X, X>), dim3(1), dim3(spec_threads(nc)), 0, s, c, spec, st);
         else
             hipLaunchKernelGGL((k_mg_coarse<X>), dim3(1), dim3(nc <= 64 ? 64 : MGC_T), 0, s, c, st);
     } else {
@@ -1198,7 +1415,7 @@ static hipError_t vcycle(hipStream_t s, const Grid& g, const MgLevelT<X, double>
         if constexpr (std::is_same_v<X, double>) {
             const long nc = long(top.nx) * top.ny * top.nz;
             if (spec)
-                hipLaunchKernelGGL((k_mg_spec<X, double>), dim3(1), dim3(nc <= 64 ? 64 : MGC_T), 0, s, top, spec, st);
+                hipLaunchKernelGGL((k_mg_spec<X, double>), dim3(1), dim3(spec_threads(nc)), 0, s, top, spec, st);
             else
                 hipLaunchKernelGGL((k_mg_coarse<X>), dim3(1), dim3(nc <= 64 ? 64 : MGC_T), 0, s, top, st);
         } else {
@@ -1281,6 +1498,8 @@ struct CycleView {
     const double* spec;
     const MgGroupCase* c;
     FieldView<X> x2;  // level 0's second vector, or null: its pairs as one pass each
+    int lmid;         // first level of the one-block bottom (mb), or last
+    MgBottomArgs<X> mb;
 };
 
 template <typename X>
@@ -1311,6 +1530,7 @@ CycleView<X> cycle_view(const MgGroupCase& gc)
     else
         v.x2 = h.x2f;
     if (v.last == 0 || v.top.ny % MP_TY != 0) v.x2 = FieldView<X>{nullptr, 0, 0};
+    v.lmid = v.last > 1 ? mg_bottom_first<X>(v.lev, v.last, v.nu, v.spec, gc.st, &v.mb) : v.last;
     return v;
 }
 
@@ -1372,9 +1592,11 @@ void group_cycle(GroupPlan& P, const std::vector<CycleView<X>>& all)
     // the coarsest solve of every case whose coarsest level is l
     for (int l = 0; l <= lmax; ++l) {
         std::vector<const CycleView<X>*> dn, dnx, co;
+        GroupItems<MgBottomArgs<X>> bt;
         for (const auto& v : all) {
-            if (l < v.last) (l == 0 && v.hx ? dnx : dn).push_back(&v);
-            if (l == v.last) co.push_back(&v);
+            if (l < v.lmid) (l == 0 && v.hx ? dnx : dn).push_back(&v);
+            if (l == v.lmid && v.lmid < v.last) bt.add(v.mb, dim3(1));
+            else if (l == v.lmid) co.push_back(&v);
         }
         if (l == 0) {
             // cases whose level 0 runs pair passes (p) and the others
@@ -1425,6 +1647,7 @@ void group_cycle(GroupPlan& P, const std::vector<CycleView<X>>& all)
             }
             P.add<MgRr<X, X, X>>(rr.v);
         }
+        P.add<MgBottom<X>>(bt.v);
         if (!co.empty()) {
             if (l == 0) {
                 // a one-level hierarchy: the coarsest solve on level 0 (FP64 only)
@@ -1454,7 +1677,7 @@ void group_cycle(GroupPlan& P, const std::vector<CycleView<X>>& all)
     for (int l = lmax - 1; l >= 0; --l) {
         std::vector<const CycleView<X>*> up, upx;
         for (const auto& v : all)
-            if (l < v.last) (l == 0 && v.hx ? upx : up).push_back(&v);
+            if (l < v.lmid) (l == 0 && v.hx ? upx : up).push_back(&v);
         if (l == 0) {
             GroupItems<typename MgProlong<X, double, X>::Args> pr;
             for (const auto* v : up) {
