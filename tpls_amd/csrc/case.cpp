@@ -1314,7 +1314,26 @@ int enqueue_pre(tpls_case* c, const StepPlan& pl)
         srcb[q] = others[0];
         dstb[q] = others[1];
     }
-    const bool lock = sizeof(T) == 4 && (c->tiling.fused & 1) && !c->timed && sor_pair3_fits(g, c->tiling);
+    // Up to HH3_CELLS every sweep and boundary kernel of the three components
+    // goes out as one launch (helmholtz3.hpp): there one component's sweep
+    // leaves much of the chip idle.  Above, three sets of planes no longer
+    // stay in L2 between neighbouring tiles.  Per step, one component's loop
+    // at a time (FP32: in lock-step with launch_sor_pair3) against three:
+    // 3.62 / 2.20 ms FP64 and 2.49 / 1.92 FP32 at 128x32x64, 6.8 / 5.2 and
+    // 4.35 / 3.90 at 256x64x128, 11.9 / 10.8 and 7.5 / 7.0 at 352x96x160,
+    // 19.9 / 18.9 and 12.9 / 12.5 at 448x128x192; with the colour sweeps
+    // split, 21.1 / 20.8 and 13.7 / 13.6 there but 29.0 / 31.6 and 19.2 / 19.6
+    // at 512x128x256.  (The passes of sor_fused bits 1 and 2 have no such
+    // form.)
+    constexpr long HH3_CELLS = 12000000;
+    // The odd pass of the three: with about one block for each CU the deep
+    // prefetch of launch_sor_odd3 is the faster (320x64x160, 264 blocks: 6.71
+    // against 6.88 ms per step FP64), with more the occupancy of
+    // launch_sor_pair3 (352x96x160, 432 blocks: 10.8 against 11.0 and, FP32,
+    // 7.04 against 7.46).
+    const bool pair3 = sor_pair3_fits(g, c->tiling) && 3L * ((g.maxl + 30) / 32) * (g.P / 8) > 320;
+    const bool small = !c->timed && !(c->tiling.fused & 6) && long(g.maxl) * g.P * g.maxn <= HH3_CELLS;
+    const bool lock = !small && sizeof(T) == 4 && (c->tiling.fused & 1) && !c->timed && sor_pair3_fits(g, c->tiling);
     const int nmin = std::min({mom[0], mom[1], mom[2]}) / 2;
     // one outer iteration of component q; three: its fused pass and the
     // boundary conditions after it are left to the three-component launch
@@ -1357,6 +1376,36 @@ int enqueue_pre(tpls_case* c, const StepPlan& pl)
         std::swap(srcb[q], dstb[q]);
         return TPLS_OK;
     };
+    if (small) {
+        FieldView<T> xs[3], xd[3], xj[3], rhs[3];
+        for (int q = 0; q < 3; ++q) rhs[q] = V(c->rhs[q]);
+        const int nits = std::max({mom[0], mom[1], mom[2]}) / 2;
+        for (int it = 1; it <= nits; ++it) {
+            if (it > nmin) {  // some of the components have finished
+                for (int q = 0; q < 3; ++q)
+                    if (it <= mom[q] / 2) RC(iteration(q, it, false));
+                continue;
+            }
+            const bool fused = it % 2 && (c->tiling.fused & 1);
+            for (int q = 0; q < 3; ++q) {
+                xs[q] = V(c->x[q][srcb[q]]);
+                xd[q] = V(c->x[q][dstb[q]]);
+                xj[q] = fused ? V(c->x[q][c->i2[q]]) : xd[q];
+            }
+            LCHK(launch_jacobi3<T>(s, g, ph, xs, rhs, V(c->mu), xj, it == 1, c->tiling));
+            LCHK(launch_helmholtz_bc3<T>(s, g, ph, xj, V(c->pres)));
+            if (fused && pair3) {
+                LCHK(launch_sor_pair3<T>(s, g, ph, xj, xd, rhs, V(c->mu), c->tiling));
+            } else if (fused) {
+                LCHK(launch_sor_odd3<T>(s, g, ph, xj, xd, rhs, V(c->mu), c->tiling));
+            } else {
+                for (int flg = 0; flg < 2; ++flg)
+                    LCHK(launch_sor3<T>(s, g, ph, xd, rhs, V(c->mu), flg, it, c->tiling));
+            }
+            LCHK(launch_helmholtz_bc3<T>(s, g, ph, xd, V(c->pres)));
+            for (int q = 0; q < 3; ++q) std::swap(srcb[q], dstb[q]);
+        }
+    }
     if (lock) {
         const int nits = std::max({mom[0], mom[1], mom[2]}) / 2;
         for (int it = 1; it <= nits; ++it) {
@@ -1393,7 +1442,7 @@ int enqueue_pre(tpls_case* c, const StepPlan& pl)
         return TPLS_OK;
     };
     for (int q = 0; q < 3; ++q) {
-        if (!lock)
+        if (!lock && !small)
             for (int it = 1; it <= mom[q] / 2; ++it) RC(iteration(q, it, false));
         RC(difference(q));
     }

@@ -163,6 +163,22 @@ hipError_t launch_helmholtz_bc(hipStream_t s, const Grid& g, const Phys& ph, int
 // launch_jacobi, launch_helmholtz_bc and launch_sor(flg 0) leave in it.
 // Needs a period divisible by 8 (jsor0_fits).
 inline bool jsor0_fits(const Grid& g) { return g.P % 8 == 0; }
+// The three components' sweeps, and their boundary conditions, as one launch
+// each (helmholtz3.hpp); launch_sor_odd3 is launch_sor_pair at an odd
+// iteration_time.
+template <typename T>
+hipError_t launch_jacobi3(hipStream_t s, const Grid& g, const Phys& ph, const FieldView<T>* xold,
+                          const FieldView<T>* rhs, FieldView<T> mu, const FieldView<T>* x, bool xold_is_zero,
+                          const Tiling& tl);
+template <typename T>
+hipError_t launch_sor3(hipStream_t s, const Grid& g, const Phys& ph, const FieldView<T>* x, const FieldView<T>* rhs,
+                       FieldView<T> mu, int flg, int iteration_time, const Tiling& tl);
+template <typename T>
+hipError_t launch_sor_odd3(hipStream_t s, const Grid& g, const Phys& ph, const FieldView<T>* xin,
+                           const FieldView<T>* xout, const FieldView<T>* rhs, FieldView<T> mu, const Tiling& tl);
+template <typename T>
+hipError_t launch_helmholtz_bc3(hipStream_t s, const Grid& g, const Phys& ph, const FieldView<T>* x,
+                                FieldView<T> pres);
 template <typename T>
 hipError_t launch_jsor0(hipStream_t s, const Grid& g, const Phys& ph, int comp, FieldView<T> xs, FieldView<T> xd,
                         FieldView<T> rhs, FieldView<T> mu, FieldView<T> pres, const Tiling& tl = Tiling{});
