@@ -18,31 +18,41 @@ __global__ void __launch_bounds__(BX* BY) k_tpls_update(Grid g, T dt, FieldView<
     phi3(i, j, k) = phi2(i, j, k) - dt * rhs;
 }
 
-// Boundary planes of a level-set field.  Pass 1, one thread per (j, k),
-// k in 1..n-1: inlet phi = z - height and outlet copy (two_phase_levelset.f90:
-// 72-82, levelset.f90:170-191).  Pass 2, one thread per (i, j), i in 0..maxl:
-// linear extrapolation to k = 0 and k = n (two_phase_levelset.f90:94-95,
-// levelset.f90:193-216).
+// Boundary planes of a level-set field: per (j, k), k in 1..n-1, inlet
+// phi = z - height and outlet copy (two_phase_levelset.f90:72-82,
+// levelset.f90:170-191), and per (i, j), i in 0..maxl, linear extrapolation to
+// k = 0 and k = n (two_phase_levelset.f90:94-95, levelset.f90:193-216).  Eleven
+// times a step, so bound by launches: the extrapolation forms the inlet and
+// outlet columns' values itself instead of waiting for them to be stored, and
+// both parts go out together, blocks [0, nbi) of x the extrapolation (2.7 us
+// at 128x32x64 against 2 x 2.65 us for a launch each).
 template <typename T>
-__global__ void k_phi_inout(Grid g, T dz, T height, FieldView<T> phi)
+__device__ __forceinline__ T phi_inlet(int k, T dz, T height)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y + 1;
-    if (k > g.maxn - 1) return;
-    T z = T(k) * dz - T(0.5) * dz;
-    phi(0, j, k) = z - height;
-    phi(g.maxl, j, k) = phi(g.maxl - 1, j, k);
+    const T z = T(k) * dz - T(0.5) * dz;
+    return z - height;
 }
 
 template <typename T>
-__global__ void k_phi_zext(Grid g, FieldView<T> phi)
+__global__ void __launch_bounds__(64) k_phi_bc(Grid g, int nbi, T dz, T height, FieldView<T> phi, int inlet_outlet)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = g.maxn, L = g.maxl;
     const int j = blockIdx.y + 1;
-    const int n = g.maxn;
-    if (i > g.maxl) return;
-    phi(i, j, 0) = T(2) * phi(i, j, 1) - phi(i, j, 2);
-    phi(i, j, n) = T(2) * phi(i, j, n - 1) - phi(i, j, n - 2);
+    if (int(blockIdx.x) >= nbi) {
+        const int k = (int(blockIdx.x) - nbi) * 64 + int(threadIdx.x) + 1;
+        if (k > n - 1) return;
+        phi(0, j, k) = phi_inlet(k, dz, height);
+        phi(L, j, k) = phi(L - 1, j, k);
+        return;
+    }
+    const int i = int(blockIdx.x) * 64 + int(threadIdx.x);
+    if (i > L) return;
+    auto at = [&](int k) {
+        if (inlet_outlet && i == 0) return phi_inlet(k, dz, height);
+        return T(phi(inlet_outlet && i == L ? L - 1 : i, j, k));
+    };
+    phi(i, j, 0) = T(2) * at(1) - at(2);
+    phi(i, j, n) = T(2) * at(n - 1) - at(n - 2);
 }
 
 // levelset.f90:44-91: sign, interface indicator and subcell distance.
@@ -403,9 +413,8 @@ hipError_t launch_tpls_update(hipStream_t s, const Grid& g, const Phys& ph, Fiel
 template <typename T>
 hipError_t launch_phi_bc(hipStream_t s, const Grid& g, double dz, double height, FieldView<T> phi, int inlet_outlet)
 {
-    if (inlet_outlet)
-        hipLaunchKernelGGL(k_phi_inout<T>, dim3((g.maxn - 1 + 63) / 64, g.P), dim3(64), 0, s, g, T(dz), T(height), phi);
-    hipLaunchKernelGGL(k_phi_zext<T>, dim3((g.maxl + 1 + 63) / 64, g.P), dim3(64), 0, s, g, phi);
+    const int nbi = (g.maxl + 1 + 63) / 64, nbk = inlet_outlet ? (g.maxn - 1 + 63) / 64 : 0;
+    hipLaunchKernelGGL(k_phi_bc<T>, dim3(nbi + nbk, g.P), dim3(64), 0, s, g, nbi, T(dz), T(height), phi, inlet_outlet);
     return hipGetLastError();
 }
 
