@@ -98,3 +98,39 @@ def test_batch_equals_alone(mode):
         assert a.diag() == b.diag()
         for f in ("u2", "v2", "w2", "phi2", "pres"):
             assert np.array_equal(a.field(f), b.field(f))
+
+
+CHILD = """
+import dataclasses, numpy as np
+from tpls_amd.case import Case, batch_step, set_batch_grouped
+from tpls_amd.config import CaseParams
+from tpls_amd.initial import make_initial
+ps = [CaseParams(nx=n, ny=16, nz=24, Re=150.0, mu_plus=2.0, dt=1e-4, noise=1e-2, seed=n) for n in (64, 48)]
+def new():
+    cs = [Case(p, precision="fp64", diagnostics=False) for p in ps]
+    for c, p in zip(cs, ps):
+        c.load(*make_initial(p))
+    return cs
+alone, both = new(), new()
+for c in alone:
+    c.step(3)
+set_batch_grouped(1)
+batch_step(both, 3)
+for a, b in zip(alone, both):
+    for f in ("u2", "phi2", "pres"):
+        x, y = a.field(f), b.field(f)
+        assert np.isfinite(x).all() and np.abs(x - y).max() <= 1e-7 * np.abs(x).max(), f
+print("solved")
+"""
+
+
+def test_second_process_on_the_device():
+    """The device may refuse cooperative launches to a second process; its
+    solves, alone and grouped, then run the streaming kernels.  Bound: twice
+    the solves' relative stopping test of 1e-10, times the condition that the
+    solutions' differences of 1e-9 have shown, with two orders to spare."""
+    import subprocess
+    import sys
+    test_iteration_limit_and_converged_guess()  # this process holds the right to them
+    r = subprocess.run([sys.executable, "-c", CHILD], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "solved" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]

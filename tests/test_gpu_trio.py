@@ -44,3 +44,16 @@ def test_three_components_in_one_launch(nx, ny, nz, mom, precision):
         for f in one:
             assert np.array_equal(one[f], three[f]), (tiles, fused, f)
     print(f"[three at once] {nx}x{ny}x{nz} {precision} {mom}", flush=True)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_above_the_largest_grid_of_the_three(precision):
+    """Past 12 M cells FP64 runs each component's loop whole and FP32 the
+    lock-step of launch_sor_pair3, with loops of different lengths."""
+    p = dataclasses.replace(BASE, nx=512, ny=128, nz=192, mom_u=8, mom_v=6, mom_w=8, ksp_pc="mg", dt=2e-5)
+    init = make_initial(p)
+    tiles = (4, 2, 8, 8, 8, 8)
+    one = fields(p, init, precision, tiles, 1, True)
+    three = fields(p, init, precision, tiles, 1, False)
+    for f in one:
+        assert np.array_equal(one[f], three[f]), f

@@ -1072,11 +1072,17 @@ int ps_enqueue_chunk(tpls_case* c)
     if (on_chip(c)) {
         CgChipLaunch l;
         RC(chip_entry(c, c->s, &l));
-        LCHK(launch_cg_chip(c->s, {l}));
-        c->ps_launched = std::max(1, c->prm.ksp_maxits);
-        LCHK(hipMemcpyAsync(c->h_cg, c->cg, sizeof(CgState), hipMemcpyDeviceToHost, c->s));
-        LCHK(hipEventRecord(c->ps_ev, c->s));
-        return TPLS_OK;
+        if (launch_cg_chip(c->s, {l}) == hipSuccess) {
+            c->ps_launched = std::max(1, c->prm.ksp_maxits);
+            LCHK(hipMemcpyAsync(c->h_cg, c->cg, sizeof(CgState), hipMemcpyDeviceToHost, c->s));
+            LCHK(hipEventRecord(c->ps_ev, c->s));
+            return TPLS_OK;
+        }
+        // Cooperative launches may be refused at any time: the device grants
+        // them to one process at once.  Nothing has run then, and the
+        // streaming kernels start from the same state.
+        (void)hipGetLastError();
+        c->chip = false;
     }
     FieldView<double> x = c->pold->view<double>(), r = c->cg_r->view<double>();
     const bool z32 = mg && c->mg.fp32;
@@ -1781,7 +1787,9 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
             chip.emplace_back();
             RC(chip_entry(c, G->s, &chip.back()));
         }
-    LCHK(launch_cg_chip(G->s, chip));
+    // refused (see ps_enqueue_chunk): those cases are solved one by one below
+    const bool refused = launch_cg_chip(G->s, chip) != hipSuccess;
+    if (refused) (void)hipGetLastError();
     LCHK(G->vc.run(G->s));
     long first = chip.size() == cs.size() ? 0 : 1, launched = 0, maxits = 1;
     for (tpls_case* c : cs) {
@@ -1818,6 +1826,16 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
         c->diag.ksp_rnorm = G->h_st[q].dp;
         c->last_its = G->h_st[q].its;
         LCHK(hipStreamWaitEvent(c->s, G->done, 0));
+        if (!refused || !on_chip(c)) continue;
+        ps_reset(c);
+        c->chip = false;
+        int rc = ps_enqueue_chunk(c);
+        for (bool fin = false; !rc && !fin;) {
+            LCHK(hipEventSynchronize(c->ps_ev));
+            rc = ps_poll(c, &fin);
+        }
+        c->chip = true;  // the group's plan holds the other cases only
+        RC(rc);
     }
     return TPLS_OK;
 }
