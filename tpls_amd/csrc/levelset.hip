@@ -24,8 +24,8 @@ __global__ void __launch_bounds__(BX* BY) k_tpls_update(Grid g, T dt, FieldView<
 // k = 0 and k = n (two_phase_levelset.f90:94-95, levelset.f90:193-216).  Eleven
 // times a step, so bound by launches: the extrapolation forms the inlet and
 // outlet columns' values itself instead of waiting for them to be stored, and
-// both parts go out together, blocks [0, nbi) of x the extrapolation (2.7 us
-// at 128x32x64 against 2 x 2.65 us for a launch each).
+// both parts go out together, blocks [0, nbi) of x the extrapolation (3.4 us
+// at 128x32x64 against 2.6 + 2.7 us for a launch each).
 template <typename T>
 __device__ __forceinline__ T phi_inlet(int k, T dz, T height)
 {
