@@ -100,6 +100,54 @@ def test_batch_equals_alone(mode):
             assert np.array_equal(a.field(f), b.field(f))
 
 
+def started(ps, refuse=0):
+    cs = [Case(p, precision="fp64") for p in ps]
+    for c, p in zip(cs, ps):
+        c.load(*make_initial(p))
+        _lib.test_refuse_chip(c, refuse)
+    return cs
+
+
+@pytest.mark.parametrize("lone", ["step", "ungrouped batch"])
+@pytest.mark.parametrize("first", ["granted", "refused"])
+def test_refused_between_grouped_steps(first, lone):
+    """The device may refuse a cooperative launch at any time: a case refused
+    in a grouped step or in one of its own is solved by the streaming kernels
+    then and in the grouped steps after it.  Each case computes what it does
+    alone when it is refused at the same step."""
+    ps = [CaseParams(nx=n, ny=14, nz=26, Re=150.0, mu_plus=2.0, seed=n, noise=1e-2) for n in (48, 65)]
+    alone, both = started(ps), started(ps)
+    if first == "refused":
+        for c in alone:
+            _lib.test_refuse_chip(c, 1)
+        for c in both:  # twice: a case that keeps its place on the chip is refused again below
+            _lib.test_refuse_chip(c, 2)
+    batch_step(both, 1)
+    for c in alone:
+        c.step(1)
+    if first == "granted":
+        assert all(map(_lib.test_on_chip, alone + both))
+        for c in alone + both:
+            _lib.test_refuse_chip(c, 1)
+    if lone == "step":
+        both[0].step(1)
+        both[1].step(1)
+    else:
+        set_batch_grouped(0)
+        try:
+            batch_step(both, 1)
+        finally:
+            set_batch_grouped(1)
+    batch_step(both, 1)
+    for c in alone:
+        c.step(2)
+    for a, b in zip(alone, both):
+        assert not _lib.test_on_chip(a) and not _lib.test_on_chip(b)
+        assert a.diag() == b.diag() and b.diag()["ksp_reason"] == 2 and b.diag()["ksp_its"] > 10
+        for f in ("u2", "v2", "w2", "phi2", "pres"):
+            assert np.array_equal(a.field(f), b.field(f)), f
+
+
 CHILD = """
 import dataclasses, numpy as np
 from tpls_amd.case import Case, batch_step, set_batch_grouped

@@ -201,3 +201,26 @@ def test_mg_apply(r, nx, ny, nz, cx, cy, cz, diag, nu):
     nl = f(nx, ny, nz, cx, cy, cz, diag, nu, r.ctypes.data, z.ctypes.data)
     check(min(nl, 0), "tpls_test_mg_apply")
     return z, nl
+
+
+def test_refuse_chip(case, n: int) -> None:
+    """Test hook: the next n launches holding the case's on-chip solve are
+    taken as refused by the device."""
+    f = lib().tpls_test_refuse_chip
+    f.argtypes = [_CASE, C.c_int]
+    check(f(case._h, n), "tpls_test_refuse_chip")
+
+
+def test_on_chip(case) -> bool:
+    """Test hook: whether the case's pressure solves run on the chip."""
+    f = lib().tpls_test_on_chip
+    f.argtypes = [_CASE]
+    return bool(f(case._h))
+
+
+def test_chip_plan(nx: int, ny: int, nz: int):
+    """Test hook: (cells per thread, threads, blocks) of the on-chip solve of
+    a grid, None for a grid that does not fit."""
+    f = lib().tpls_test_chip_plan
+    out = (C.c_int * 3)()
+    return None if f(nx, ny, nz, out) else tuple(out)

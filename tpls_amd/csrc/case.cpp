@@ -169,6 +169,7 @@ struct tpls_case {
     CgChipCase* chip_d = nullptr;
     void* chip_ws = nullptr;
     unsigned chip_epoch = 1;
+    int chip_refuse = 0;         // launches still to be taken as refused (tpls_test_refuse_chip)
     double* h_out = nullptr;   // pinned host mirror of red_out
     tpls_diag diag{};
     long steps_done = 0;
@@ -1059,6 +1060,21 @@ int chip_entry(tpls_case* c, hipStream_t s, CgChipLaunch* out)
     return TPLS_OK;
 }
 
+// launch_cg_chip of these cases' solves; as if the device had refused it where
+// a test asks for that (tpls_test_refuse_chip).
+hipError_t chip_launch(hipStream_t s, const std::vector<tpls_case*>& cs, const std::vector<CgChipLaunch>& l)
+{
+    bool refuse = false;
+    for (tpls_case* c : cs)
+        if (c->chip_refuse > 0) {
+            --c->chip_refuse;
+            refuse = true;
+        }
+    const hipError_t e = refuse ? hipErrorCooperativeLaunchTooLarge : launch_cg_chip(s, l);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 // A solve on the chip that waited too long for another block.
 int chip_check(const CgState& st)
 {
@@ -1072,7 +1088,7 @@ int ps_enqueue_chunk(tpls_case* c)
     if (on_chip(c)) {
         CgChipLaunch l;
         RC(chip_entry(c, c->s, &l));
-        if (launch_cg_chip(c->s, {l}) == hipSuccess) {
+        if (chip_launch(c->s, {c}, {l}) == hipSuccess) {
             c->ps_launched = std::max(1, c->prm.ksp_maxits);
             LCHK(hipMemcpyAsync(c->h_cg, c->cg, sizeof(CgState), hipMemcpyDeviceToHost, c->s));
             LCHK(hipEventRecord(c->ps_ev, c->s));
@@ -1081,7 +1097,6 @@ int ps_enqueue_chunk(tpls_case* c)
         // Cooperative launches may be refused at any time: the device grants
         // them to one process at once.  Nothing has run then, and the
         // streaming kernels start from the same state.
-        (void)hipGetLastError();
         c->chip = false;
     }
     FieldView<double> x = c->pold->view<double>(), r = c->cg_r->view<double>();
@@ -1598,7 +1613,7 @@ int step_impl(tpls_case* c)
 int g_batch_grouped = 1;
 
 struct SolveGroup {
-    std::vector<uint64_t> key;        // the cases' uids, in batch order
+    std::vector<uint64_t> key;        // in batch order: the cases' uids, and whether each is solved on the chip
     std::vector<double> coef;         // their level-0 coefficients
     GroupPlan vc, it[2], gather;      // first V-cycle; iteration by p parity; state gather
     GroupPlan hh;                     // this step's Helmholtz loops and solve set-up
@@ -1641,7 +1656,10 @@ std::vector<double> group_coef(const std::vector<tpls_case*>& cs)
 int group_for(const std::vector<tpls_case*>& cs, SolveGroup** out)
 {
     std::vector<uint64_t> key;
-    for (tpls_case* c : cs) key.push_back(c->uid);
+    for (tpls_case* c : cs) {
+        key.push_back(c->uid);
+        key.push_back(on_chip(c));  // the tables leave those cases out
+    }
     const std::vector<double> coef = group_coef(cs);
     if (t_group && t_group->key == key && t_group->coef == coef) {
         *out = t_group.get();
@@ -1782,14 +1800,15 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
     }
     LCHK(G->hh.run(G->s));
     std::vector<CgChipLaunch> chip;
+    std::vector<tpls_case*> chip_cs;
     for (tpls_case* c : cs)
         if (on_chip(c)) {
             chip.emplace_back();
             RC(chip_entry(c, G->s, &chip.back()));
+            chip_cs.push_back(c);
         }
     // refused (see ps_enqueue_chunk): those cases are solved one by one below
-    const bool refused = launch_cg_chip(G->s, chip) != hipSuccess;
-    if (refused) (void)hipGetLastError();
+    const bool refused = chip_launch(G->s, chip_cs, chip) != hipSuccess;
     LCHK(G->vc.run(G->s));
     long first = chip.size() == cs.size() ? 0 : 1, launched = 0, maxits = 1;
     for (tpls_case* c : cs) {
@@ -1820,22 +1839,25 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
     LCHK(hipEventRecord(G->done, G->s));
     for (int q = 0; q < G->n; ++q) {
         tpls_case* c = cs[q];
+        LCHK(hipStreamWaitEvent(c->s, G->done, 0));
+        if (refused && on_chip(c) && !G->h_st[q].done) {
+            c->chip = false;  // from the next step on in the group's tables
+            ps_reset(c);
+            int rc = ps_enqueue_chunk(c);
+            for (bool fin = false; !rc && !fin;) {
+                LCHK(hipEventSynchronize(c->ps_ev));
+                rc = ps_poll(c, &fin);
+            }
+            RC(rc);
+            continue;
+        }
+        // every way out of an iteration sets done
+        if (!G->h_st[q].done) return fail(TPLS_ERR_HIP, "a pressure solve of the group did not run");
         *c->h_cg = G->h_st[q];
         c->diag.ksp_its = G->h_st[q].its;
         c->diag.ksp_reason = G->h_st[q].reason;
         c->diag.ksp_rnorm = G->h_st[q].dp;
         c->last_its = G->h_st[q].its;
-        LCHK(hipStreamWaitEvent(c->s, G->done, 0));
-        if (!refused || !on_chip(c)) continue;
-        ps_reset(c);
-        c->chip = false;
-        int rc = ps_enqueue_chunk(c);
-        for (bool fin = false; !rc && !fin;) {
-            LCHK(hipEventSynchronize(c->ps_ev));
-            rc = ps_poll(c, &fin);
-        }
-        c->chip = true;  // the group's plan holds the other cases only
-        RC(rc);
     }
     return TPLS_OK;
 }
@@ -2677,6 +2699,30 @@ int tpls_test_fail_next_step(tpls_case* c)
 {
     if (!c) return fail(TPLS_ERR_ARG, "null case");
     c->fail_next = 1;
+    return TPLS_OK;
+}
+
+// Test hooks, not part of the public interface: the next n launches that hold
+// the case's on-chip solve are taken as refused by the device (host-side:
+// nothing is launched); whether the case's solves run on the chip; and the
+// boxes of a grid's solve there (cells per thread, threads, blocks), or
+// TPLS_ERR_ARG for a grid that does not fit.
+int tpls_test_refuse_chip(tpls_case* c, int n)
+{
+    if (!c) return fail(TPLS_ERR_ARG, "null case");
+    c->chip_refuse = n;
+    return TPLS_OK;
+}
+
+int tpls_test_on_chip(const tpls_case* c) { return c && on_chip(c) ? 1 : 0; }
+
+int tpls_test_chip_plan(int nx, int ny, int nz, int* out)
+{
+    CgChipPlan p{};
+    if (!out || !cg_chip_plan(nx, ny, nz, &p)) return fail(TPLS_ERR_ARG, "no plan");
+    out[0] = p.cells;
+    out[1] = p.threads;
+    out[2] = p.nblk;
     return TPLS_OK;
 }
 
