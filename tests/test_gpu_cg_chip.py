@@ -100,6 +100,42 @@ def test_batch_equals_alone(mode):
             assert np.array_equal(a.field(f), b.field(f))
 
 
+def test_largest_iteration_limit():
+    """A solve after one that stopped at its first iteration, both with the
+    largest ksp_maxits: its reductions carry numbers of their own.  (The right
+    side is an eigenvector of the operator, so one iteration solves it.)"""
+    rng = np.random.default_rng(6)
+    nx, ny, nz = 48, 14, 26
+    L, M, N, h = nx + 1, ny + 1, nz + 1, 1.0 / nz
+    u3, inlet = np.zeros((L + 1, M + 1, N - 1), order="F"), np.zeros(N - 1)
+    eig = np.zeros((L + 1, M + 1, N + 1), order="F")
+    eig[:] = np.cos(np.pi * (np.arange(L + 1) - 0.5) / nx)[:, None, None]
+    rhs = np.asfortranarray(rng.standard_normal(eig.shape))
+
+    def solve(b, maxits):
+        pres = np.zeros_like(eig)
+        return pres, _lib.pressure_solve(pres, b, u3, inlet, L, M, N, h, h, h, 1e-4, 1e-8, 1e-50, 1e5, maxits)
+
+    want, info = solve(rhs, 10000)
+    assert info[2] == 2 and info[0] > 10
+    for _ in range(3):
+        assert solve(eig, 2 ** 31 - 1)[1][::2] == (1, 2)
+        got, again = solve(rhs, 2 ** 31 - 1)
+        assert again == info and np.array_equal(got, want)
+
+
+def test_reduction_numbers_wrap():
+    """Numbers that pass 2^32 within a solve change nothing."""
+    p = CaseParams(nx=48, ny=14, nz=26, Re=150.0, mu_plus=2.0, seed=3, noise=1e-2)
+    a, b = started([p, p])
+    _lib.test_chip_epoch(b, 2 ** 32 - 21)
+    for c in (a, b):
+        c.step(2)
+    assert a.diag() == b.diag() and a.diag()["ksp_its"] > 11
+    for f in ("u2", "pres"):
+        assert np.array_equal(a.field(f), b.field(f))
+
+
 def started(ps, refuse=0):
     cs = [Case(p, precision="fp64") for p in ps]
     for c, p in zip(cs, ps):

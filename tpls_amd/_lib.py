@@ -211,6 +211,13 @@ def test_refuse_chip(case, n: int) -> None:
     check(f(case._h, n), "tpls_test_refuse_chip")
 
 
+def test_chip_epoch(case, epoch: int) -> None:
+    """Test hook: number the case's next on-chip reduction."""
+    f = lib().tpls_test_chip_epoch
+    f.argtypes = [_CASE, C.c_uint]
+    check(f(case._h, epoch), "tpls_test_chip_epoch")
+
+
 def test_on_chip(case) -> bool:
     """Test hook: whether the case's pressure solves run on the chip."""
     f = lib().tpls_test_on_chip

@@ -162,13 +162,15 @@ struct tpls_case {
     CgState* cg = nullptr;
     CgState* h_cg = nullptr;   // pinned host mirror
     // the plain CG on the chip (cg_chip.hip): its boxes, device table and
-    // workspace, and the number of the next solve's first reduction
+    // workspace, the number of the next solve's first reduction, and whether
+    // a solve has been launched whose end has not been seen
     bool chip = false;
     CgChipPlan chip_plan{};
     CgChipCase chip_h{};         // the table's contents
     CgChipCase* chip_d = nullptr;
     void* chip_ws = nullptr;
     unsigned chip_epoch = 1;
+    bool chip_ran = false;
     int chip_refuse = 0;         // launches still to be taken as refused (tpls_test_refuse_chip)
     double* h_out = nullptr;   // pinned host mirror of red_out
     tpls_diag diag{};
@@ -1055,8 +1057,13 @@ int chip_entry(tpls_case* c, hipStream_t s, CgChipLaunch* out)
         LCHK(hipMemcpyAsync(c->chip_d, &c->chip_h, sizeof k, hipMemcpyHostToDevice, s));
         LCHK(hipStreamSynchronize(s));
     }
+    if (c->chip_ran) {
+        // a solve that failed: how many reductions it made is not known
+        LCHK(hipMemsetAsync(c->chip_ws, 0, cg_chip_slot_bytes(p), s));
+        c->chip_epoch = 1;
+    }
     *out = {&c->chip_plan, c->chip_d, c->chip_epoch};
-    c->chip_epoch += 2 * unsigned(std::max(1, c->prm.ksp_maxits)) + 2;
+    c->chip_ran = true;
     return TPLS_OK;
 }
 
@@ -1075,10 +1082,17 @@ hipError_t chip_launch(hipStream_t s, const std::vector<tpls_case*>& cs, const s
     return e;
 }
 
-// A solve on the chip that waited too long for another block.
-int chip_check(const CgState& st)
+// After a solve on the chip: the error of one that waited too long for another
+// block, else the next solve's numbers follow on from this one's reductions.
+// (Numbers that leave some out could meet a word of an earlier solve again
+// after 2^32 of them; these meet none but their predecessors.)
+int chip_done(tpls_case* c, const CgState& st)
 {
-    return st.pad ? fail(TPLS_ERR_HIP, "the pressure solve's blocks waited too long for each other") : int(TPLS_OK);
+    if (!c->chip_ran) return TPLS_OK;
+    if (st.pad) return fail(TPLS_ERR_HIP, "the pressure solve's blocks waited too long for each other");
+    c->chip_ran = false;
+    c->chip_epoch += 2 * unsigned(st.its);
+    return TPLS_OK;
 }
 
 int ps_enqueue_chunk(tpls_case* c)
@@ -1097,7 +1111,7 @@ int ps_enqueue_chunk(tpls_case* c)
         // Cooperative launches may be refused at any time: the device grants
         // them to one process at once.  Nothing has run then, and the
         // streaming kernels start from the same state.
-        c->chip = false;
+        c->chip = c->chip_ran = false;
     }
     FieldView<double> x = c->pold->view<double>(), r = c->cg_r->view<double>();
     const bool z32 = mg && c->mg.fp32;
@@ -1203,7 +1217,7 @@ int ps_poll(tpls_case* c, bool* finished)
         int rc = harvest_events(c);
         if (rc) return rc;
     }
-    RC(chip_check(*c->h_cg));
+    RC(chip_done(c, *c->h_cg));
     if (c->h_cg->done || c->ps_launched >= c->prm.ksp_maxits) {
         c->diag.ksp_its = c->h_cg->its;
         c->diag.ksp_reason = c->h_cg->reason;
@@ -1830,7 +1844,7 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
         LCHK(hipEventSynchronize(G->ev));
         bool all = true;
         for (int q = 0; q < G->n; ++q) {
-            RC(chip_check(G->h_st[q]));
+            RC(chip_done(cs[q], G->h_st[q]));
             if (!on_chip(cs[q]) && !G->h_st[q].done && launched < cs[q]->prm.ksp_maxits) all = false;
         }
         if (all) break;
@@ -2711,6 +2725,14 @@ int tpls_test_refuse_chip(tpls_case* c, int n)
 {
     if (!c) return fail(TPLS_ERR_ARG, "null case");
     c->chip_refuse = n;
+    return TPLS_OK;
+}
+
+// The number of the case's next on-chip reduction.
+int tpls_test_chip_epoch(tpls_case* c, unsigned epoch)
+{
+    if (!c) return fail(TPLS_ERR_ARG, "null case");
+    c->chip_epoch = epoch;
     return TPLS_OK;
 }
 

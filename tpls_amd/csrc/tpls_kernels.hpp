@@ -255,7 +255,9 @@ struct CgChipArgs {
 struct CgChipLaunch {
     const CgChipPlan* plan;
     const CgChipCase* dev;
-    unsigned epoch;  // the solve's first reduction; it numbers two per iteration
+    // number of the solve's first reduction: one more than that of the last
+    // reduction whose words are in the slots (two per iteration, modulo 2^32)
+    unsigned epoch;
 };
 bool cg_chip_plan(int nx, int ny, int nz, CgChipPlan* out);
 bool cg_chip_fits_device(const CgChipPlan& p);
