@@ -100,6 +100,33 @@ def test_batch_equals_alone(mode):
             assert np.array_equal(a.field(f), b.field(f))
 
 
+@pytest.mark.parametrize("mode", [1, 2])
+def test_batch_of_more_than_one_launch(mode):
+    """More cases of one segment length than a launch takes, in all several
+    blocks for each CU, of different block shapes."""
+    sizes = [(20 + q % 3, 8 + 2 * (q % 4), 12 + q % 5) for q in range(61)] + [(64, 16, 32)] * 6 + [(48, 12, 24)] * 5
+    ps = [CaseParams(nx=n[0], ny=n[1], nz=n[2], Re=150.0, mu_plus=2.0, seed=q, noise=1e-2, mom_u=2, mom_v=2, mom_w=2,
+                     levelset_its=2) for q, n in enumerate(sizes)]
+    plans = [_lib.test_chip_plan(*n) for n in sizes]
+    for cells in {p[0] for p in plans}:
+        print(cells, "cells:", sum(p[0] == cells for p in plans), "cases", sum(p[2] for p in plans if p[0] == cells))
+    assert sum(p[2] for p in plans) > 2 * 256
+    alone, both = started(ps), started(ps)
+    for c in alone:
+        c.step(2)
+    set_batch_grouped(mode)
+    try:
+        batch_step(both, 2)
+    finally:
+        set_batch_grouped(1)
+    for a, b in zip(alone, both):
+        assert a.diag() == b.diag()
+        for f in ("u2", "v2", "w2", "phi2", "pres"):
+            assert np.array_equal(a.field(f), b.field(f))
+        a.close()
+        b.close()
+
+
 def test_largest_iteration_limit():
     """A solve after one that stopped at its first iteration, both with the
     largest ksp_maxits: its reductions carry numbers of their own.  (The right
