@@ -31,8 +31,8 @@
 // alternate between two buffers: one is written again only after every block
 // has stored a word that follows its loads of it.
 //
-// Per iteration, before and after: 128x32x64 22 -> 7.5 us, 150x46x77 30 ->
-// 8.6, 256x64x128 57 -> 11.5.  Of the 8.6 (20,700 cycles) the two waits for
+// Per iteration, before and after: 128x32x64 22 -> 7.1 us, 150x46x77 30 ->
+// 8.6, 256x64x128 57 -> 12.0.  Of the 8.6 (20,700 cycles) the two waits for
 // the other blocks' sums take about 10,000, the stencil and the updates the
 // rest: the latency of a word's way from one XCD to another bounds it.
 //
@@ -498,12 +498,15 @@ size_t chip_lds(const CgChipPlan& p)
 // The boxes of a grid: a function of its extents only, so that a case sums in
 // the same order alone and in any batch.  Of all partitions into at most
 // CG_CHIP_BLOCKS boxes that the registers and LDS of a block hold, the one
-// with the least estimated cycles per iteration beyond the fixed ones (about
-// 11,000): 50 per wavefront and cell (LDS and FP64), 300 per round of halo
-// cells, 900 per 64 blocks polled.  Measured cycles per iteration (cells per
-// thread, blocks): 128x32x64 17,400 (4, 64), 18,200 (2, 128), 17,900 (1, 256),
-// 20,100 (8, 64); 150x46x77 20,700 (4, 192), 24,400 (8, 120), 26,800 (16, 125);
-// 256x64x128 27,700 (16, 256), 29,300 (8, 256).
+// with the least estimated ns per iteration beyond the fixed 4,000: 22 per
+// wavefront and cell (LDS and FP64), 80 per wavefront, 100 per cell of a
+// segment (the chain of its column), 100 per round of halo cells, 600 per 64
+// blocks polled.  Fitted to 200 partitions of 17 grids, 6 % rms.  Measured us
+// per iteration (cells per thread, blocks; the chosen one first): 64x16x32 5.0
+// (2, 64), 5.3 (1, 64), 5.8 (4, 64), 6.0 (2, 128); 96x22x41 6.4 (2, 126), 6.8
+// (2, 64), 6.8 (1, 192); 128x32x64 7.1 (4, 128), 7.6 (2, 128), 7.4 (4, 64), 8.0
+// (8, 128); 150x46x77 8.3 (4, 192), 9.4 (8, 190), 10.2 (16, 192); 179x42x192
+// 11.5 (8, 252), 12.0 (16, 252); 256x64x128 11.9 (16, 256), 12.9 (8, 256).
 bool cg_chip_plan(int nx, int ny, int nz, CgChipPlan* out)
 {
     if (long(nx) * ny * nz > long(CG_CHIP_BLOCKS) * chip_threads(24) * 24) return false;
@@ -537,11 +540,11 @@ bool cg_chip_plan(int nx, int ny, int nz, CgChipPlan* out)
                     p.lds = chip_lds(p);
                     if (p.lds > CG_CHIP_LDS) continue;
                     const double waves = double((need + 63) / 64);
-                    // registers: 8 cells at 16 wavefronts spill a little, 24 a lot
-                    const double spill = cells == 24 ? 4.0 : (cells == 8 ? 1.1 : 1.0);
-                    const double cost = 50.0 * spill * waves * cells +
-                                        300.0 * ((p.fstride + p.threads - 1) / p.threads) +
-                                        900.0 * ((p.nblk + 63) / 64);
+                    // registers: 8 cells spill a little, 24 a lot
+                    const double spill = cells == 24 ? 4.0 : (cells == 8 ? 1.25 : 1.0);
+                    const double cost = 22.0 * spill * waves * cells + 80.0 * waves + 100.0 * cells +
+                                        100.0 * ((p.fstride + p.threads - 1) / p.threads) +
+                                        600.0 * ((p.nblk + 63) / 64);
                     if (best < 0.0 || cost < best) {
                         best = cost;
                         *out = p;
