@@ -1,6 +1,6 @@
 """The plain CG solve as one launch (cg_chip.hip): boxes of every segment
-length, with remainders in each direction, at the smallest grids and on either
-side of the largest one that fits.  The bound is the solve's own stopping
+length (1, 2, 4, 8, 16 and 24 cells), with remainders in each direction, at the
+smallest grids and on either side of the largest one that fits.  The bound is the solve's own stopping
 test, evaluated in numpy; FP64 rounding of the two residuals is far below it."""
 import numpy as np
 import pytest
@@ -215,6 +215,26 @@ def test_refused_between_grouped_steps(first, lone):
             assert np.array_equal(a.field(f), b.field(f)), f
 
 
+@pytest.mark.parametrize("nx,ny,nz", [(33, 18, 29), (96, 22, 41), (150, 46, 77), (5, 4, 8)])
+def test_streaming_solve(nx, ny, nz):
+    """The streaming kernels of a case whose launch is refused, on grids that
+    otherwise run on the chip.  Both solutions have residuals below their
+    stopping test, so their difference (mean-free) is at most the sum of the
+    residuals over the smallest eigenvalue; the recurrences' residuals are
+    within a tenth of the true ones."""
+    p = CaseParams(nx=nx, ny=ny, nz=nz, Re=150.0, mu_plus=2.0, seed=nz, noise=1e-2, height=0.47)
+    chip, stream = started([p]) + started([p], refuse=1)
+    for c in (chip, stream):
+        c.step(1)
+    assert _lib.test_on_chip(chip) and not _lib.test_on_chip(stream)
+    a, b = chip.diag(), stream.diag()
+    assert a["ksp_reason"] == b["ksp_reason"] == 2 and abs(a["ksp_its"] - b["ksp_its"]) <= 2 + 0.05 * b["ksp_its"]
+    low = min(2 - 2 * np.cos(np.pi / nx), 2 - 2 * np.cos(2 * np.pi / ny), 2 - 2 * np.cos(np.pi / nz)) * nz ** 2
+    x, y = (c.field("pres_old")[1:nx + 1, 1:ny + 1, 1:nz + 1] for c in (chip, stream))
+    assert np.isfinite(x).all() and np.linalg.norm(x) > 0
+    assert np.linalg.norm(x - y) <= 1.1 * (a["ksp_rnorm"] + b["ksp_rnorm"]) / low + 1e-12 * np.linalg.norm(x)
+
+
 CHILD = """
 import dataclasses, numpy as np
 from tpls_amd.case import Case, batch_step, set_batch_grouped
@@ -235,17 +255,21 @@ for a, b in zip(alone, both):
     for f in ("u2", "phi2", "pres"):
         x, y = a.field(f), b.field(f)
         assert np.isfinite(x).all() and np.abs(x - y).max() <= 1e-7 * np.abs(x).max(), f
-print("solved")
+from tpls_amd import _lib
+print("solved", "on the chip" if all(map(_lib.test_on_chip, alone + both)) else "by streaming kernels")
 """
 
 
 def test_second_process_on_the_device():
-    """The device may refuse cooperative launches to a second process; its
-    solves, alone and grouped, then run the streaming kernels.  Bound: twice
-    the solves' relative stopping test of 1e-10, times the condition that the
-    solutions' differences of 1e-9 have shown, with two orders to spare."""
+    """A second process solves rightly, alone and grouped, whether the device
+    grants it cooperative launches or not.  (What a refusal leads to is shown
+    by test_refused_between_grouped_steps and test_streaming_solve; the child
+    says which it met.)  Bound: twice the solves' relative stopping test of
+    1e-10, times the condition that the solutions' differences of 1e-9 have
+    shown, with two orders to spare."""
     import subprocess
     import sys
     test_iteration_limit_and_converged_guess()  # this process holds the right to them
     r = subprocess.run([sys.executable, "-c", CHILD], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "solved" in r.stdout, r.stdout[-1000:] + r.stderr[-2000:]
+    print(r.stdout.strip().splitlines()[-1])
