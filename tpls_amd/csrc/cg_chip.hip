@@ -31,8 +31,8 @@
 // alternate between two buffers: one is written again only after every block
 // has stored a word that follows its loads of it.
 //
-// Per iteration, before and after: 128x32x64 22 -> 7.1 us, 150x46x77 30 ->
-// 8.6, 256x64x128 57 -> 12.0.  Of the 8.6 (20,700 cycles) the two waits for
+// Per iteration, before and after: 128x32x64 22 -> 6.9 us, 150x46x77 30 ->
+// 8.3, 256x64x128 57 -> 11.8.  Of 150x46x77's (20,700 cycles) the two waits for
 // the other blocks' sums take about 10,000, the stencil and the updates the
 // rest: the latency of a word's way from one XCD to another bounds it.
 //
@@ -176,16 +176,19 @@ __global__ void __launch_bounds__(chip_threads(C)) k_cg_chip(CgChipArgs args)
     // cells whose loads are in flight together: all at once, the loads of a
     // long segment would spill the cells' own registers
     constexpr int GROUP = C == 8 ? 2 : 4;
-    // the block's case: the last of those that start at or before it
-    int lo = 0;
-    for (int hi = args.n; hi - lo > 1;) {
-        const int mid = (lo + hi) / 2;
-        if (int(blockIdx.x) >= args.b0[mid]) lo = mid;
-        else hi = mid;
-    }
-    const unsigned epoch = args.epoch[lo];
-    const int first = args.b0[lo];
-    const CgChipCase a = *args.c[lo];
+    // the block's case (unrolled: with a search at run time the registers that
+    // the solve's loop gets cost 256x64x128 1.5 % of its time)
+    const CgChipCase* ap = args.c[0];
+    unsigned epoch = args.epoch[0];
+    int first = 0;
+#pragma unroll
+    for (int q = 1; q < CG_CHIP_MAX; ++q)
+        if (q < args.n && int(blockIdx.x) >= args.b0[q]) {
+            ap = args.c[q];
+            epoch = args.epoch[q];
+            first = args.b0[q];
+        }
+    const CgChipCase a = *ap;
     CgState* const st = a.st;
     if (st->done) return;
     const int b = int(blockIdx.x) - first, t = threadIdx.x, nthr = blockDim.x;

@@ -230,7 +230,7 @@ hipError_t launch_cg_x(hipStream_t s, const Grid& g, const Phys& ph, FieldView<d
 // ---- the plain CG of a grid that fits on the chip, one launch (cg_chip.hip) ----
 constexpr int CG_CHIP_BLOCKS = 256;         // boxes at most: one block per CU
 constexpr size_t CG_CHIP_LDS = 152 * 1024;  // p and its halo
-constexpr int CG_CHIP_MAX = 64;             // cases per launch
+constexpr int CG_CHIP_MAX = 32;             // cases per launch
 struct CgChipPlan {
     int cells, threads, nseg, nblk, fstride;
     int bx, by, bz, gx, gy, gz;  // box extents and counts
