@@ -1,5 +1,5 @@
 // Launchers of the Helmholtz sweeps (helmholtz_ops.hpp), one component at a
-// time and grouped over the cases of a batch; helmholtz3.hip launches the
+// time and grouped over the cases of a batch; helmholtz3.hpp launches the
 // three components together.
 #include <memory>
 

@@ -865,7 +865,11 @@ static int spec_threads(long cells) { return int(std::min<long>(MGS_T, (cells + 
 //
 // One launch instead of about (4 nu + 2) (n - 1) + 1.  With the vectors in
 // memory each of the about 28 passes waited for the L2: 48 us for levels of
-// 4096, 512 and 64 cells in FP64, 24 us now.  What is left is the
+// 4096, 512 and 64 cells in FP64, 24 us now.  Levels that the LDS does not hold
+// (28 B a cell in FP64, 16 in FP32, and the levels below) stay with the
+// multi-block kernels: of 64x32x32 in FP64, whose level 1 has 8192 cells, a
+// cycle's kernels took 146 us with that level in the block's memory passes and
+// take 101 now (FP32, in LDS: 131 and 84).  What is left is the
 // first level's sweeps (one CU's FP64 rate) and, in every pass, the latency
 // of LDS and a barrier.  All levels run the same code, loops not unrolled: a
 // pass unrolled per level spent more on instruction-cache misses than on
