@@ -215,6 +215,29 @@ def test_refused_between_grouped_steps(first, lone):
             assert np.array_equal(a.field(f), b.field(f)), f
 
 
+@pytest.mark.parametrize("refused", [0, 2])
+def test_refused_in_part(refused):
+    """A refusal of the second of a group's launches leaves the first one's
+    cases solved and on the chip; one of the first launch refuses them all."""
+    sizes = [(48, 14, 26), (50, 12, 24), (96, 22, 41)]
+    cells = [_lib.test_chip_plan(*n)[0] for n in sizes]
+    assert cells[0] == cells[1] != cells[2]  # two launches
+    ps = [CaseParams(nx=n[0], ny=n[1], nz=n[2], Re=150.0, mu_plus=2.0, seed=n[0], noise=1e-2) for n in sizes]
+    alone, both = started(ps), started(ps)
+    _lib.test_refuse_chip(both[refused], 1)
+    for q in range(3) if refused == 0 else [2]:
+        _lib.test_refuse_chip(alone[q], 1)
+    for _ in range(2):
+        batch_step(both, 1)
+        for a, b in zip(alone, both):
+            a.step(1)
+            assert _lib.test_on_chip(a) == _lib.test_on_chip(b)
+            assert a.diag() == b.diag()
+            for f in ("u2", "phi2", "pres"):
+                assert np.array_equal(a.field(f), b.field(f)), f
+    assert [_lib.test_on_chip(b) for b in both] == ([False] * 3 if refused == 0 else [True, True, False])
+
+
 @pytest.mark.parametrize("nx,ny,nz", [(33, 18, 29), (96, 22, 41), (150, 46, 77), (5, 4, 8)])
 def test_streaming_solve(nx, ny, nz):
     """The streaming kernels of a case whose launch is refused, on grids that

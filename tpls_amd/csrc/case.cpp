@@ -1062,24 +1062,10 @@ int chip_entry(tpls_case* c, hipStream_t s, CgChipLaunch* out)
         LCHK(hipMemsetAsync(c->chip_ws, 0, cg_chip_slot_bytes(p), s));
         c->chip_epoch = 1;
     }
-    *out = {&c->chip_plan, c->chip_d, c->chip_epoch};
+    *out = {&c->chip_plan, c->chip_d, c->chip_epoch, c->chip_refuse > 0};
+    if (out->refuse) --c->chip_refuse;
     c->chip_ran = true;
     return TPLS_OK;
-}
-
-// launch_cg_chip of these cases' solves; as if the device had refused it where
-// a test asks for that (tpls_test_refuse_chip).
-hipError_t chip_launch(hipStream_t s, const std::vector<tpls_case*>& cs, const std::vector<CgChipLaunch>& l)
-{
-    bool refuse = false;
-    for (tpls_case* c : cs)
-        if (c->chip_refuse > 0) {
-            --c->chip_refuse;
-            refuse = true;
-        }
-    const hipError_t e = refuse ? hipErrorCooperativeLaunchTooLarge : launch_cg_chip(s, l);
-    if (e != hipSuccess) (void)hipGetLastError();
-    return e;
 }
 
 // After a solve on the chip: the error of one that waited too long for another
@@ -1102,7 +1088,7 @@ int ps_enqueue_chunk(tpls_case* c)
     if (on_chip(c)) {
         CgChipLaunch l;
         RC(chip_entry(c, c->s, &l));
-        if (chip_launch(c->s, {c}, {l}) == hipSuccess) {
+        if (launch_cg_chip(c->s, {l}) == hipSuccess) {
             c->ps_launched = std::max(1, c->prm.ksp_maxits);
             LCHK(hipMemcpyAsync(c->h_cg, c->cg, sizeof(CgState), hipMemcpyDeviceToHost, c->s));
             LCHK(hipEventRecord(c->ps_ev, c->s));
@@ -1111,6 +1097,7 @@ int ps_enqueue_chunk(tpls_case* c)
         // Cooperative launches may be refused at any time: the device grants
         // them to one process at once.  Nothing has run then, and the
         // streaming kernels start from the same state.
+        (void)hipGetLastError();
         c->chip = c->chip_ran = false;
     }
     FieldView<double> x = c->pold->view<double>(), r = c->cg_r->view<double>();
@@ -1814,15 +1801,15 @@ int group_solve(const std::vector<tpls_case*>& cs, int mode)
     }
     LCHK(G->hh.run(G->s));
     std::vector<CgChipLaunch> chip;
-    std::vector<tpls_case*> chip_cs;
     for (tpls_case* c : cs)
         if (on_chip(c)) {
             chip.emplace_back();
             RC(chip_entry(c, G->s, &chip.back()));
-            chip_cs.push_back(c);
         }
-    // refused (see ps_enqueue_chunk): those cases are solved one by one below
-    const bool refused = chip_launch(G->s, chip_cs, chip) != hipSuccess;
+    // refused (see ps_enqueue_chunk), all of it or from some launch on: the
+    // cases not solved are solved one by one below
+    const bool refused = launch_cg_chip(G->s, chip) != hipSuccess;
+    if (refused) (void)hipGetLastError();
     LCHK(G->vc.run(G->s));
     long first = chip.size() == cs.size() ? 0 : 1, launched = 0, maxits = 1;
     for (tpls_case* c : cs) {

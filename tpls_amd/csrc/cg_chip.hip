@@ -585,9 +585,9 @@ size_t cg_chip_face_bytes(const CgChipPlan& p) { return size_t(2) * p.nblk * p.f
 // order, same segment length).  Beyond one block for each CU the set grows as
 // long as the device holds the blocks at once: small grids have small blocks,
 // and the launches of a large batch run one after another.  Grouped step of
-// 64 cases of 64x16x32: 40.6 ms with at most 256 blocks a launch, 28.8 so, 30.5
-// by streaming kernels that all cases share; of 16 such cases 11.8, 9.1 and
-// 12.0.
+// 64 cases of 64x16x32: 40.6 ms with at most 256 blocks a launch, 26.6 so, 30.5
+// by streaming kernels that all cases share; of 16 such cases 11.8, 7.9 and
+// 12.0.  An error leaves the cases of the launches before it solved.
 hipError_t launch_cg_chip(hipStream_t s, const std::vector<CgChipLaunch>& cases)
 {
     // the blocks of this shape that the device holds
@@ -607,6 +607,7 @@ hipError_t launch_cg_chip(hipStream_t s, const std::vector<CgChipLaunch>& cases)
         CgChipArgs a{};
         int blocks = 0, threads = 0;
         size_t lds = 0;
+        bool refuse = false;
         for (size_t q = f; q < cases.size() && a.n < CG_CHIP_MAX; ++q) {
             const CgChipPlan& p = *cases[q].plan;
             if (done[q] || p.cells != cases[f].plan->cells) continue;
@@ -620,8 +621,10 @@ hipError_t launch_cg_chip(hipStream_t s, const std::vector<CgChipLaunch>& cases)
             blocks += p.nblk;
             threads = t;
             lds = l;
+            refuse = refuse || cases[q].refuse;
             done[q] = 1;
         }
+        if (refuse) return hipErrorCooperativeLaunchTooLarge;
         void* argv[] = {&a};
         const hipError_t e = with_cells(cases[f].plan->cells, [&](auto k) {
             return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(k), dim3(blocks), dim3(threads), argv,

@@ -258,6 +258,7 @@ struct CgChipLaunch {
     // number of the solve's first reduction: one more than that of the last
     // reduction whose words are in the slots (two per iteration, modulo 2^32)
     unsigned epoch;
+    bool refuse;  // take the launch as refused by the device (tests)
 };
 bool cg_chip_plan(int nx, int ny, int nz, CgChipPlan* out);
 bool cg_chip_fits_device(const CgChipPlan& p);
